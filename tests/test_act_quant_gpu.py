@@ -52,3 +52,28 @@ def test_fp8_indexer_from_quantised_inputs(dsa, dev):
     # Against the unquantised bf16 inputs the fp8 rounding stays small.
     full = ref.indexer_logits(qf, kf, w, None, sparse_mode=3)
     assert ((got[fin] - full[fin]).abs().mean() / full[fin].abs().mean()).item() < 0.1
+
+
+@pytest.mark.parametrize("xdtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,rows", [(8, 262149), (64, 3), (72, 65), (128, 32769), (136, 129), (264, 17), (520, 5), (1032, 3),
+                                    (2056, 2), (4104, 3), (8200, 2),
+                                    (16392, 1)])
+def test_rows_in_lane_groups_bit_exact(dsa, dev, n, rows, xdtype):
+    """Both sides of every group width and register count of the aligned rows (16-byte chunks: 8 bf16
+    or 4 fp32), one and several rows per group, with signed zeros, tiny, huge and infinite values: the
+    oracle divides in IEEE fp32, so codes and scales are equal bit for bit."""
+    g = torch.Generator().manual_seed(n + rows)
+    x = torch.randn((rows, n), generator=g) * torch.exp2(torch.randint(-30, 30, (rows, 1), generator=g).float())
+    x[0, ::3], x[0, 1::3] = -0.0, 1e-30
+    x[-1, 0] = float("inf")
+    x = x.to(xdtype)
+    for dtype in (torch.int8, torch.float8_e4m3fn):
+        y, s = dsa.act_quant(x.to(dev), dtype=dtype)
+        wy, ws = ref.act_quant(x, dtype=dtype)
+        assert torch.equal(s.cpu(), ws)
+        keep = slice(0, rows - 1)  # the infinite row's quotients hold inf / inf: codes below, against the wave-per-row kernel
+        assert torch.equal(y[keep].cpu().view(torch.uint8), wy[keep].view(torch.uint8))
+        pad = torch.zeros(rows * n + 1, dtype=xdtype)
+        pad[1:] = x.flatten()
+        z, _ = dsa.act_quant(pad.to(dev)[1:].view(rows, n), dtype=dtype)  # rows off 16 bytes: the other kernel
+        assert torch.equal(y.view(torch.uint8), z.view(torch.uint8))
