@@ -194,3 +194,18 @@ def test_lightning_indexer_long_context_topk(dsa, dev):
     idx, _ = dsa.lightning_indexer(qd, kd, wd, key_scale=ksd, sparse_count=K, sparse_mode=3)
     ri, _ = ref.topk_stable(logits.view(S1, S2).float().cpu(), K)
     assert torch.equal(idx.view(S1, K).cpu(), ri)
+
+
+@pytest.mark.parametrize("H", [32, 33, 47, 48, 49, 63, 64])
+@pytest.mark.parametrize("D,S1", [(128, 70), (64, 70), (128, 2)])
+def test_fp8_head_reduction_each_head(dsa, dev, H, D, S1):
+    """Row t weights head t % H alone, so its logits are that head's ReLU'd scores: a head met by
+    another head's weight, counted twice or left out is off by whole scores (32 and 33 heads: the dense
+    and the sparse reduction; 2 rows: the key split).  Held to the module's bar (the matrix cores'
+    own sums of 128 fp8 products are not exact enough near zero for a bound from f16 rounding alone)."""
+    q, k, _, ks = _inputs(1, S1, 200, H, D, torch.float8_e4m3fn, seed=H * D + S1)
+    w = torch.zeros(1, S1, H)
+    head = torch.arange(S1) % H
+    w[0, torch.arange(S1), head] = 1.0
+    got = dsa.indexer_logits(q.to(dev), k.unsqueeze(2).to(dev), w.to(dev), ks.to(dev), sparse_mode=0).cpu()
+    _assert_logits(got, ref.indexer_logits(q, k, w, ks, sparse_mode=0))

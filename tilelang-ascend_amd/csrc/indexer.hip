@@ -25,7 +25,8 @@
 // (v_cvt_pk_f16_f32 ... clamp), and form the B operand of a 16x16x32 f16 MFMA
 // whose A operand holds the token's 32 head weights (f16, times the heads'
 // scales and a per-token power of two) in every row: every row of the result
-// is sum_h w[h] ReLU(S[h][key]), accumulated in fp32, two MFMAs per 64 heads.  bf16/fp16 inputs (unbounded scores): fp32 ReLU,
+// is sum_h w[h] ReLU(S[h][key]), accumulated in fp32 (more than 32 heads: one
+// structured-sparse 16x16x64 MFMA, sparse_sum).  bf16/fp16 inputs (unbounded scores): fp32 ReLU,
 // multiply by w[t, h], sum the lane's 4 head rows, then two cross-lane adds
 // over the 4 row groups.  After four 16-key slices lane l holds key l of the
 // 64-key tile, so each token's logits go out as one coalesced 256-byte store.
@@ -159,13 +160,14 @@ __device__ __forceinline__ int head_score_exponent(float l1) {
 // every component.  In: `w` the fp32 weights of heads 16 hb + 4g + i (lane
 // (g, r)), scaled in place to W_h = w_h 2^e_h.  Out: `codes` byte hb = the E8M0
 // code 127 - e_h of head 16 hb + r (lane (g, r)'s A row); `wa` = W as the f16
-// A operands of the head-reduction MFMAs (block pairs (0, 1) and (2, 3)),
-// normalised by a power of two so that max |W| lies in [2^14, 2^15); `post`
+// A operand of the head-reduction MFMA (blocks 0 and 1), normalised by a power of two so that max |W| lies in [2^14, 2^15); `post`
 // undoes that power at the store.  kFixed: every e_h = 25, which bounds any
 // e4m3 row (the sample pass, whose logits only place the filter thresholds).
-template <int kD, bool kFixed>
+// kSparse: `wa` holds the token's A operand of sparse_sum instead (kTok: its
+// rows), the lanes' weights passed on through `wl`, 64 floats of LDS of this wave.
+template <int kD, bool kFixed, bool kSparse, int kTok>
 __device__ __forceinline__ void fp8_head_scales(const Operand<kFp8, kD> (&qa)[4], f32x4 (&w)[4], int nhb,
-                                                uint32_t& codes, u32x4 (&wa)[2], float& post) {
+                                                uint32_t& codes, u32x4& wa, float& post, float* wl) {
   Operand<kFp8, kD> ones;
   if constexpr (Operand<kFp8, kD>::kWhole) {
 #pragma unroll
@@ -204,11 +206,24 @@ __device__ __forceinline__ void fp8_head_scales(const Operand<kFp8, kD> (&qa)[4]
   const float up = __uint_as_float((uint32_t)(127 + 14 - e) << 23);
   // m, and with it post, is the same in every lane (lane (g, r) saw the weights of heads 4g + i + 16 hb).
   post = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(127 + e - 14) << 23)));
+  if constexpr (kSparse) {
+    const int lane = threadIdx.x & (kWave - 1), r = lane & 15, g = lane >> 4;
+    if (r == 0) {
 #pragma unroll
-  for (int pr = 0; pr < 2; ++pr)
-    wa[pr] = u32x4{pack_f16x2(w[2 * pr].x * up, w[2 * pr].y * up), pack_f16x2(w[2 * pr].z * up, w[2 * pr].w * up),
-                   pack_f16x2(w[2 * pr + 1].x * up, w[2 * pr + 1].y * up),
-                   pack_f16x2(w[2 * pr + 1].z * up, w[2 * pr + 1].w * up)};
+      for (int hb = 0; hb < 4; ++hb) *reinterpret_cast<f32x4*>(wl + 16 * hb + 4 * g) = w[hb] * up;
+    }
+    __builtin_amdgcn_wave_barrier();
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int head = 16 * (2 * (g >> 1) + (e & 3) / 2) + 4 * (2 * (g & 1) + e / 4) + 2 * (r & 1) + (e & 1);
+      v[e] = ((r >> 1) & 1) == kTok ? wl[head] : 0.f;
+    }
+    wa = u32x4{pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3]), pack_f16x2(v[4], v[5]), pack_f16x2(v[6], v[7])};
+    return;
+  }
+  wa = u32x4{pack_f16x2(w[0].x * up, w[0].y * up), pack_f16x2(w[0].z * up, w[0].w * up),
+             pack_f16x2(w[1].x * up, w[1].y * up), pack_f16x2(w[1].z * up, w[1].w * up)};
 }
 
 // B operand of the head-reduction MFMA for head blocks hb0, hb1: lane (g, r)
@@ -216,6 +231,28 @@ __device__ __forceinline__ void fp8_head_scales(const Operand<kFp8, kD> (&qa)[4]
 // (i < 4) as its K = 8g .. 8g+7.
 __device__ __forceinline__ u32x4 relu_operand(const f32x4& c0, const f32x4& c1) {
   return u32x4{relu_f16x2(c0.x, c0.y), relu_f16x2(c0.z, c0.w), relu_f16x2(c1.x, c1.y), relu_f16x2(c1.z, c1.w)};
+}
+
+// Head reduction of more than 32 heads by one structured-sparse MFMA: D +=
+// W * relu(scores) over K = 64 heads in the cycles a dense 16x16x32 takes for 32
+// (the dense pair took a fifth of the matrix cycles, and these passes run at the
+// card's power limit: 4096 rows x 32768 keys with top-2048 990 -> 960 us, x 131072
+// keys 3550 -> 3370 us).  W has at most two weights in every four K: even rows hold heads 4m, 4m + 1 of each four, odd rows heads 4m + 2, 4m + 3
+// (sparse_index), so a logit is the sum of an even and an odd row.  Rows 4n + 2j
+// and 4n + 2j + 1 belong to the wave's token j: both tokens accumulate into one D,
+// whose components 2j, 2j + 1 in every lane are token j's halves for key r.
+// Operands (lane (g, r)): B element 4 hb + i is the score of head 16 hb + 4g + i
+// of key r; A element e of row r meets B half g / 2 (blocks 2 (g / 2) + (e % 4) /
+// 2) of lane group 2 (g % 2) + e / 4 (checked on the device by one-hot operands).
+typedef _Float16 f16x16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ int sparse_index(int r) { return (r & 1) ? (int)0xEEEEEEEEu : 0x44444444; }
+__device__ __forceinline__ f32x4 sparse_sum(const u32x4& w, const f32x4& c0, const f32x4& c1, const f32x4& c2,
+                                            const f32x4& c3, const f32x4& d, int index) {
+  const u32x4 lo = relu_operand(c0, c1), hi = relu_operand(c2, c3);
+  typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
+  const u32x8 b = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+  return __builtin_amdgcn_smfmac_f32_16x16x64_f16(__builtin_bit_cast(f16x8, w), __builtin_bit_cast(f16x16, b), d, index,
+                                                  0, 0);
 }
 
 struct IdxArgs {
@@ -405,9 +442,12 @@ __device__ __forceinline__ void indexer_body(const IdxArgs& a) {
   // the block pair (hb0, hb1) = (0, 1) or (2, 3), as in relu_operand -- built
   // with the per-head score scales once q has arrived (fp8_head_scales).
   constexpr bool kMfmaSum = kKind == kFp8;
+  constexpr bool kSparseSum = kMfmaSum && kNhb > 2;
+  static_assert(!kSparseSum || kTokPW <= 2, "two tokens' rows in one accumulator");
+  const int spidx = sparse_index(r);
   Operand<kKind, kD> qa[kTokPW][4];
   f32x4 wv[kTokPW][4];
-  u32x4 wa[kTokPW][2];
+  u32x4 wa[kTokPW];
   float post[kTokPW];
 #pragma unroll
   for (int j = 0; j < kTokPW; ++j) {
@@ -599,7 +639,16 @@ __device__ __forceinline__ void indexer_body(const IdxArgs& a) {
 #pragma unroll
   for (int j = 0; j < kTokPW; ++j) {
     qscale[j] = 0x7f7f7f7fu;
-    if constexpr (kMfmaSum) fp8_head_scales<kD, kMode == kModeSample>(qa[j], wv[j], nhb, qscale[j], wa[j], post[j]);
+  }
+  if constexpr (kSparseSum) {
+    __shared__ __align__(16) float wlds[kIdxWaves][kTokPW][64];
+    fp8_head_scales<kD, kMode == kModeSample, true, 0>(qa[0], wv[0], nhb, qscale[0], wa[0], post[0], wlds[wave][0]);
+    if constexpr (kTokPW == 2)
+      fp8_head_scales<kD, kMode == kModeSample, true, 1>(qa[1], wv[1], nhb, qscale[1], wa[1], post[1], wlds[wave][1]);
+  } else if constexpr (kMfmaSum) {
+#pragma unroll
+    for (int j = 0; j < kTokPW; ++j)
+      fp8_head_scales<kD, kMode == kModeSample, false, 0>(qa[j], wv[j], nhb, qscale[j], wa[j], post[j], nullptr);
   }
   if (ntiles > 0) commit(Slot0{}, 0);
   if constexpr (kUL) {
@@ -639,24 +688,33 @@ __device__ __forceinline__ void indexer_body(const IdxArgs& a) {
       const int sub = kSplit ? wave : si;
       Operand<kKind, kD> kb;
       load_operand_lds<kKind, kD>(kb, &ktile[buf][(sub * 16 + r) * kPitch + g * kLB]);
+      if constexpr (kSparseSum) {
+        f32x4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < kTokPW; ++j) {
+          const f32x4 c0 = mfma_qk<kKind, kD, 0>(qa[j][0], kb, qscale[j]);
+          const f32x4 c1 = mfma_qk<kKind, kD, 1>(qa[j][1], kb, qscale[j]);
+          const f32x4 c2 = mfma_qk<kKind, kD, 2>(qa[j][2], kb, qscale[j]);
+          const f32x4 c3 = kNhb > 3 ? mfma_qk<kKind, kD, 3>(qa[j][3], kb, qscale[j]) : f32x4{0.f, 0.f, 0.f, 0.f};
+          d = sparse_sum(wa[j], c0, c1, c2, c3, d, spidx);
+          // Tokens in turn: interleaved, their scores do not fit three waves' registers.
+          if constexpr (!kSplit) __builtin_amdgcn_sched_barrier(0);
+        }
+        res[0] = (kSplit || g == sub) ? d.x + d.y : res[0];
+        if constexpr (kTokPW == 2) res[1] = (kSplit || g == sub) ? d.z + d.w : res[1];
+        continue;
+      }
 #pragma unroll
       for (int j = 0; j < kTokPW; ++j) {
         if constexpr (kMfmaSum) {
           // sum_h w[h] ReLU(S[h][key]) on the matrix cores: A = w in every row,
           // B = the ReLU'd scores, so every row of D holds key r's logit.
-          f32x4 d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int pr = 0; pr < 2; ++pr) {
-            if (2 * pr < nhb) {
-              const f32x4 c0 = pr == 0 ? mfma_qk<kKind, kD, 0>(qa[j][0], kb, qscale[j])
-                                       : mfma_qk<kKind, kD, 2>(qa[j][2], kb, qscale[j]);
-              const f32x4 c1 = 2 * pr + 1 >= nhb ? f32x4{0.f, 0.f, 0.f, 0.f}
-                               : pr == 0        ? mfma_qk<kKind, kD, 1>(qa[j][1], kb, qscale[j])
-                                                : mfma_qk<kKind, kD, 3>(qa[j][3], kb, qscale[j]);
-              d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, wa[j][pr]),
-                                                         __builtin_bit_cast(f16x8, relu_operand(c0, c1)), d, 0, 0, 0);
-            }
-          }
+          // Up to 32 heads (more: sparse_sum above).
+          const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+          const f32x4 c0 = mfma_qk<kKind, kD, 0>(qa[j][0], kb, qscale[j]);
+          const f32x4 c1 = nhb > 1 ? mfma_qk<kKind, kD, 1>(qa[j][1], kb, qscale[j]) : zero;
+          const f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+              __builtin_bit_cast(f16x8, wa[j]), __builtin_bit_cast(f16x8, relu_operand(c0, c1)), zero, 0, 0, 0);
           res[j] = (kSplit || g == sub) ? d.x : res[j];
         } else {
           float acc2[2] = {0.f, 0.f};  // two chains: head blocks 0, 2 and 1, 3
