@@ -27,9 +27,9 @@
 // scales and a per-token power of two) in every row: every row of the result
 // is sum_h w[h] ReLU(S[h][key]), accumulated in fp32 (more than 32 heads: one
 // structured-sparse 16x16x64 MFMA, sparse_sum).  bf16/fp16 inputs (unbounded scores): fp32 ReLU,
-// multiply by w[t, h], sum the lane's 4 head rows, then two cross-lane adds
-// over the 4 row groups.  After four 16-key slices lane l holds key l of the
-// 64-key tile, so each token's logits go out as one coalesced 256-byte store.
+// multiply by w[t, h], sum the lane's 4 head rows; the sums of a tile's four
+// slices go over the 4 row groups together (group_sums).  After four 16-key
+// slices lane l holds key l of the 64-key tile, so each token's logits go out as one coalesced 256-byte store.
 #include <algorithm>
 
 #include "common.hpp"
@@ -253,6 +253,20 @@ __device__ __forceinline__ f32x4 sparse_sum(const u32x4& w, const f32x4& c0, con
   const u32x8 b = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
   return __builtin_amdgcn_smfmac_f32_16x16x64_f16(__builtin_bit_cast(f16x8, w), __builtin_bit_cast(f16x16, b), d, index,
                                                   0, 0);
+}
+
+// Sums over the four lane groups of four values per lane: lane group g gets the sum of x[g].  Three
+// swaps and three adds on the VALU for a token's 64 keys, where each 16-key slice took two LDS
+// shuffles and a select (packed bf16 rows, 24 heads, top-2048 included: 560 -> 523 us).
+__device__ __forceinline__ float group_sums(const float (&x)[4]) {
+  // permlane32_swap(a, b): {a.lo, b.lo} and {a.hi, b.hi}; permlane16_swap the same by odd and even groups.
+  auto add32 = [](float a, float b) {
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+  };
+  const float y0 = add32(x[0], x[2]), y1 = add32(x[1], x[3]);
+  const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(y0), __float_as_uint(y1), false, false);
+  return __uint_as_float(s[0]) + __uint_as_float(s[1]);
 }
 
 struct IdxArgs {
@@ -681,6 +695,7 @@ __device__ __forceinline__ void indexer_body(const IdxArgs& a) {
     }
 
     float res[kTokPW];
+    float part[kTokPW][4];  // bf16 / fp16: the lane's head sums of each 16-key slice
 #pragma unroll
     for (int j = 0; j < kTokPW; ++j) res[j] = 0.f;
 #pragma unroll
@@ -729,11 +744,15 @@ __device__ __forceinline__ void indexer_body(const IdxArgs& a) {
               acc = fmaf(wv[j][hb].w, relu(c.w), acc);
             }
           }
-          float acc = acc2[0] + acc2[1];
-          acc += __shfl_xor(acc, 16, kWave);
-          acc += __shfl_xor(acc, 32, kWave);
-          res[j] = (kSplit || g == sub) ? acc : res[j];
+          part[j][si] = acc2[0] + acc2[1];
         }
+      }
+    }
+    if constexpr (!kMfmaSum) {
+#pragma unroll
+      for (int j = 0; j < kTokPW; ++j) {
+        if constexpr (kSplit) part[j][1] = part[j][2] = part[j][3] = part[j][0];  // one slice: its sum in every group
+        res[j] = group_sums(part[j]);
       }
     }
     // kUL, kSplit: the next tile goes to LDS before this one's stores, so that
