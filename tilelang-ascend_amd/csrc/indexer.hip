@@ -940,11 +940,16 @@ static IdxArgs make_idx_args(const void* q, const void* k, const float* k_scale,
   return a;
 }
 
-// Keys per workgroup: enough workgroups to fill 256 CUs several times over.
-// split: one token per workgroup (dense logits of few query rows).
+// Keys per workgroup.  3072 workgroups are four whole rounds of the three a CU
+// holds, and level out batches of unequal lengths, whose grid spans the longest
+// (packed bf16 rows of 340 to 1699 queries by 3000 to 15000 keys: 523 -> 464 us
+// against 2048 workgroups; 4096 rows by 8192 keys 322 -> 311; 4096 and more
+// workgroups gain nothing further and cost the latter 10%).  split: one token
+// per workgroup (dense logits of few query rows), 2048: their chunks are short
+// already (32 rows by 131072 keys).
 static int64_t indexer_key_chunk(int64_t B, int64_t S1, int64_t S2, bool split = false) {
   const int64_t tok_groups = B * (split ? S1 : (S1 + 7) / 8);
-  const int64_t chunks = (2048 + tok_groups - 1) / tok_groups;
+  const int64_t chunks = ((split ? 2048 : 3072) + tok_groups - 1) / tok_groups;
   int64_t chunk = (S2 + chunks - 1) / chunks;
   chunk = ((chunk + kIdxKeyTile - 1) / kIdxKeyTile) * kIdxKeyTile;
   return chunk < 1024 ? 1024 : chunk;
