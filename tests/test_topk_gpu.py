@@ -239,3 +239,23 @@ def test_candidates_across_zero(dsa, dev):
     _check(dsa, dev, x, 2048)
     _check(dsa, dev, x, 333)
     _check(dsa, dev, x[:, :9000], 2048)
+
+
+@pytest.mark.parametrize("n", [1027, 4097, 5001, 8191, 15001, 16386, 32767])
+@pytest.mark.parametrize("shift", [0, 1, 3])
+def test_rows_off_16_bytes(dsa, dev, n, shift):
+    """Rows that start on any dword (an odd leading dimension, a shifted first row) through the
+    register path's 16-byte loads: every register chunk count, each remainder of the last group,
+    with and without row lengths, bit-exact."""
+    rows, ld, k = 7, n + 2 - n % 2 - 1, 700
+    g = torch.Generator().manual_seed(n + shift)
+    buf = torch.randn(rows * ld + shift, generator=g)
+    x = buf[shift:].view(rows, ld)[:, :n]
+    lens = torch.tensor([n, n - 1, n - 2, n - 3, 4, 1, 0], dtype=torch.int32)
+    xd = buf.to(dev)[shift:].view(rows, ld)[:, :n]
+    for rl in (None, lens):
+        masked = x if rl is None else torch.where(torch.arange(n) < rl.view(-1, 1), x, float("-inf"))
+        want, wv = ref.topk_stable(masked, k)
+        idx, val = dsa.topk_selector(xd, k, row_len=None if rl is None else rl.to(dev), return_values=True)
+        assert torch.equal(idx.cpu(), want)
+        assert torch.equal(val.cpu(), wv)
