@@ -257,6 +257,24 @@ int dsa_sparse_mla_fwd_noalloc(int kind, const void* q, const void* kv, const in
                                int64_t block_size, int64_t max_blocks, int64_t topk, float sm_scale, int is_causal,
                                void* out, float* lse, void* stream);
 
+/* 1 when dsa_sparse_mla_decode_parts takes this shape: at most 8 query rows,
+ * 1024 (row, head) pairs and 2048 slots. */
+int dsa_sparse_mla_decode_parts_applies(int64_t B, int64_t S, int64_t H, int64_t topk);
+
+/*
+ * dsa_sparse_mla_fwd for decode rows whose latent and rope parts lie apart, as
+ * the torch_npu-style decode entry passes them
+ * (examples/sparse_flash_attention/bench_sfa/sparse_flash_attn_pa_no_cv_pipeline.py:384-419,
+ * which joins them first): q [B, S, H, 512] with q_rope [B, S, H, 64], kv rows
+ * of 512 with kv_rope rows of 64 in the same row space; every part 16-byte
+ * aligned.  Other arguments, workspace and result as dsa_sparse_mla_fwd.
+ */
+int dsa_sparse_mla_decode_parts(int kind, const void* q, const void* q_rope, const void* kv, const void* kv_rope,
+                                const int32_t* indices, const int32_t* block_table, const int32_t* actual_q_len,
+                                const int32_t* actual_kv_len, int64_t B, int64_t S, int64_t H, int64_t Skv,
+                                int64_t block_size, int64_t max_blocks, int64_t topk, float sm_scale, int is_causal,
+                                void* out, float* lse, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Workspace bytes dsa_sparse_attention_fwd needs (0 for d_qk 128, and when no split is used). */
 size_t dsa_sparse_attention_workspace_size(int64_t B, int64_t S, int64_t H, int64_t kv_group, int64_t d_qk,
                                            int64_t topk);

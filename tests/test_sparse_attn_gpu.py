@@ -248,3 +248,30 @@ def test_torch_op_equals_wrapper(dsa, dev):
     assert torch.equal(o.cpu(), _run(dsa, dev, q, kv, sink, idx, 512 ** -0.5))
     assert torch.equal(l.cpu(), _lse(dsa, dev, q, kv, sink, idx, 512 ** -0.5))
 
+
+@pytest.mark.parametrize("T,N,topk,nb", [(1, 16, 40, 3), (3, 48, 300, 20), (8, 128, 2048, 21)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_decode_parts_equal_the_joined_call(dsa, dev, T, N, topk, nb, dtype):
+    """Latent and rope parts read where they lie against sparse_mla_fwd on their joined rows: bit-equal
+    (one workgroup per row, chunks with a ragged last one, the largest shape; -1 slots, a key length)."""
+    g = torch.Generator().manual_seed(T * N + topk)
+    bs = 128
+    q, qr = torch.randn(T, N, 512, generator=g).to(dtype), torch.randn(T, N, 64, generator=g).to(dtype)
+    k, kr = (torch.randn(nb, bs, 1, d, generator=g).to(dtype) for d in (512, 64))
+    idx = torch.stack([torch.randperm(nb * bs, generator=g)[:topk] for _ in range(T)]).to(torch.int32)
+    idx[:, 1::7] = -1
+    bt = torch.randperm(nb, generator=g).to(torch.int32).view(1, nb)
+    ql, kl = torch.tensor([T], dtype=torch.int32), torch.tensor([nb * bs - 5], dtype=torch.int32)
+    q, qr, k, kr, idx, bt, ql, kl = (x.to(dev) for x in (q, qr, k, kr, idx, bt, ql, kl))
+    for mode in (0, 3):
+        out = dsa.sparse_attn_tilelang(q, k, k, idx.view(T, 1, topk), 0.05, 1, ql, kl, query_rope=qr, key_rope=kr,
+                                       sparse_mode=mode, block_table=bt)
+        want, _ = dsa.sparse_mla_fwd(torch.cat((q, qr), -1).unsqueeze(0), torch.cat((k, kr), -1),
+                                     idx.view(1, T, 1, topk), 0.05, block_table=bt, actual_seq_lengths_query=ql,
+                                     actual_seq_lengths_kv=kl, is_causal=mode == 3)
+        assert torch.equal(out, want[0])
+        # A transposed query layout cannot be read in place: the joined call takes it, same result.
+        qt = q.transpose(0, 1).contiguous().transpose(0, 1)
+        same = dsa.sparse_attn_tilelang(qt, k, k, idx.view(T, 1, topk), 0.05, 1, ql, kl, query_rope=qr, key_rope=kr,
+                                        sparse_mode=mode, block_table=bt)
+        assert torch.equal(out, same)

@@ -33,6 +33,12 @@ hipError_t launch_sparse_gqa(int is_fp16, const void* q, const void* kv, const i
                              int64_t Skv, int64_t topk, float sm_scale, int causal, void* out, float* lse,
                              hipStream_t stream);
 size_t sparse_mla_workspace_bytes(int64_t tokens, int64_t H, int64_t topk);
+bool mla_decode_applies(int64_t T, int64_t H, int64_t topk);
+hipError_t launch_mla_decode_rows(int is_fp16, const void* q, const void* q_rope, const void* kv, const void* kv_rope,
+                                  const int32_t* indices, const int32_t* block_table, const int32_t* q_len,
+                                  const int32_t* kv_len, int64_t B, int64_t S, int64_t G, int64_t H, int64_t Skv,
+                                  int64_t block_size, int64_t max_blocks, int64_t topk, float sm_scale, int causal,
+                                  void* out, float* lse, void* workspace, hipStream_t stream);
 size_t mla_scratch_bytes();
 hipError_t mla_scratch_ptr(void** out);
 size_t v4_workspace_bytes(int64_t T, int64_t H, int64_t cap, bool out_f32);
@@ -343,6 +349,37 @@ size_t dsa_sparse_attention_workspace_size(int64_t B, int64_t S, int64_t H, int6
   if (B <= 0 || S <= 0 || H <= 0 || topk <= 0 || kv_group <= 0 || H % kv_group != 0) return 0;
   if (d_qk != 576) return 0;  // the 128-wide kernel needs no workspace
   return dsa::sparse_mla_workspace_bytes(B * S * kv_group, H / kv_group, topk);
+}
+
+int dsa_sparse_mla_decode_parts_applies(int64_t B, int64_t S, int64_t H, int64_t topk) {
+  return B >= 1 && S >= 1 && H >= 16 && topk >= 1 && B <= kMaxInt && S <= kMaxInt && H % 16 == 0 && H <= 1024 &&
+         dsa::mla_decode_applies(B * S, H, topk);
+}
+
+int dsa_sparse_mla_decode_parts(int kind, const void* q, const void* q_rope, const void* kv, const void* kv_rope,
+                                const int32_t* indices, const int32_t* block_table, const int32_t* actual_q_len,
+                                const int32_t* actual_kv_len, int64_t B, int64_t S, int64_t H, int64_t Skv,
+                                int64_t block_size, int64_t max_blocks, int64_t topk, float sm_scale, int is_causal,
+                                void* out, float* lse, void* workspace, size_t workspace_bytes, void* stream) {
+  if (kind != DSA_KIND_BF16 && kind != DSA_KIND_FP16) return reject("sparse_mla_decode_parts: kind must be bf16 or fp16");
+  if (!dsa_sparse_mla_decode_parts_applies(B, S, H, topk))
+    return reject("sparse_mla_decode_parts: at most 8 query rows, 1024 (row, head) pairs and 2048 slots");
+  if (block_table) {
+    if (block_size <= 0 || max_blocks <= 0 || block_size * max_blocks > kMaxInt)
+      return reject("sparse_mla_decode_parts: paged kv needs block_size > 0 and max_blocks > 0");
+  } else if (Skv < 0 || Skv > kMaxInt) {
+    return reject("sparse_mla_decode_parts: bad Skv");
+  }
+  if (!(sm_scale > 0.f) || !(sm_scale < 3.0e38f))
+    return reject("sparse_mla_decode_parts: sm_scale must be positive and finite");
+  if (workspace_bytes < dsa_sparse_mla_workspace_size(B, S, H, topk))
+    return reject("sparse_mla_decode_parts: workspace too small");
+  if (!q || !q_rope || !kv || !kv_rope || !indices || !out || !lse)
+    return reject("sparse_mla_decode_parts: null pointer");
+  const int64_t skv_eff = block_table ? block_size * max_blocks : Skv;
+  return ok(dsa::launch_mla_decode_rows(kind == DSA_KIND_FP16, q, q_rope, kv, kv_rope, indices, block_table, actual_q_len,
+                                        actual_kv_len, B, S, 1, H, skv_eff, block_size, max_blocks, topk, sm_scale,
+                                        is_causal ? 1 : 0, out, lse, workspace, static_cast<hipStream_t>(stream)));
 }
 
 int dsa_sparse_attention_fwd(int kind, const void* q, const void* kv, const int32_t* indices,

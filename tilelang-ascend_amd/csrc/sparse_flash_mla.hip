@@ -188,8 +188,9 @@ constexpr int dec_lds() {
 
 struct DecArgs {
   const uint16_t* q;      // [T, H, 512]
+  const uint16_t* q_rope; // [T, H, 64] (kMode 5)
   const uint8_t* kv;      // rows of 1 KB
-  const uint8_t* kv2;     // rows tagged kCmpTag, or null
+  const uint8_t* kv2;     // rows tagged kCmpTag, or null; kMode 5: the rows' 128-byte tails
   const int32_t* rows;    // [T, cap]
   const int32_t* count;   // [T]; -1: padded row
   const float* sinks;     // [H] or null
@@ -309,7 +310,10 @@ __device__ __forceinline__ short dec_round(float p, float& back) {
 // here), 4 sparse MLA index rows (kD = 576: K is the whole row, V its first 512).
 template <bool kF16, int kMode, int kD = 512>
 __global__ __launch_bounds__(256) void v4_decode_rows_kernel(DecArgs a) {
-  static_assert(kD == 512 || (kD == 576 && kMode == 4), "576-wide rows: sparse MLA index rows");
+  // kMode 4 and 5: sparse MLA index rows (576 wide); 5: q and kv hold the 512
+  // latent dims alone, the 64-dim tails lie in q_rope and kv2.
+  constexpr bool kMla = kMode >= 4, kTails = kMode == 5;
+  static_assert(kD == (kMla ? 576 : 512), "576-wide rows: sparse MLA index rows");
   constexpr int kBlkLds = dec_blk_lds<kD>();
   constexpr int kSteps = kD / 32;                      // Q K^T steps of 32 dims
   constexpr int kDmaPerBlk = kD == 576 ? kDecBlk + 2 : kDecBlk;  // DMA instructions per block
@@ -323,13 +327,17 @@ __global__ __launch_bounds__(256) void v4_decode_rows_kernel(DecArgs a) {
   const int s_lo = blockIdx.z * a.chunk;  // this workgroup's slots: s_lo .. s_lo + chunk - 1
   // Q^T operands: head h0 + r, dims 32 st + 8g .. +7 (loaded first: they need no row list).
   u32x4 qb[kSteps];
-  const uint16_t* qp = a.q + ((int64_t)t * a.H + h0 + r) * kD + 8 * g;
+  const int64_t qrow = (int64_t)t * a.H + h0 + r;
+  const uint16_t* qp = a.q + qrow * (kTails ? 512 : kD) + 8 * g;
 #pragma unroll
-  for (int st = 0; st < kSteps; ++st) qb[st] = *reinterpret_cast<const u32x4*>(qp + 32 * st);
+  for (int st = 0; st < kSteps; ++st) {
+    const uint16_t* src = kTails && st >= 16 ? a.q_rope + qrow * 64 + 8 * g + 32 * (st - 16) : qp + 32 * st;
+    qb[st] = *reinterpret_cast<const u32x4*>(src);
+  }
   int cnt_raw, vb = 0, vnw = 0, vw0 = 0, thr = 0, nread = 0;
   const V4Args& v = a.v4;
-  int mb = 0, mg = 0, mkl = 0, mlim = 0;  // kMode 4: batch, KV group, kv length, causal bound of the row
-  if constexpr (kMode == 4) {
+  int mb = 0, mg = 0, mkl = 0, mlim = 0;  // kMla: batch, KV group, kv length, causal bound of the row
+  if constexpr (kMla) {
     // A row past its batch's query length has no valid slot (out 0, lse -inf, as
     // the gather kernel gives it); a slot is valid iff 0 <= idx < kv_len and, when
     // causal, idx <= kv_len - q_len + s.
@@ -402,7 +410,7 @@ __global__ __launch_bounds__(256) void v4_decode_rows_kernel(DecArgs a) {
   auto row_of = [&](int i) -> int32_t {
     if constexpr (kMode == 0) {
       return rowl[i];
-    } else if constexpr (kMode == 4) {
+    } else if constexpr (kMla) {
       const int idx = a.mla.idx[(int64_t)t * a.cap + i];
       const bool ok = idx >= 0 && idx < mkl && idx <= mlim;
       if (a.mla.block_table) {
@@ -493,13 +501,13 @@ __global__ __launch_bounds__(256) void v4_decode_rows_kernel(DecArgs a) {
     const bool valid = rows >= 0 && slot_of(k) < cnt;
     const uint32_t vmask = (uint32_t)(__builtin_amdgcn_ballot_w64(valid) >> (16 * j)) & 0xffffu;
     const int32_t rz = valid ? rows : 0;  // empty slots read row 0 (their scores are masked)
-    constexpr int kRowBytes = kD * 2;
+    constexpr int kRowBytes = kTails ? 1024 : kD * 2;
 #pragma unroll
     for (int u = 0; u < kDecBlk; ++u) {
       const int ru = __builtin_amdgcn_readlane(rz, 16 * j + u);
-      // Index rows (kMode 4) use all 31 bits; V4 lists tag compressed rows.
-      const uint8_t* base = (kMode != 4 && (ru & kCmpTag)) ? a.kv2 : a.kv;
-      const int64_t pr = kMode == 4 ? (int64_t)ru : (int64_t)(ru & ~kCmpTag);
+      // Index rows (kMla) use all 31 bits; V4 lists tag compressed rows.
+      const uint8_t* base = (!kMla && (ru & kCmpTag)) ? a.kv2 : a.kv;
+      const int64_t pr = kMla ? (int64_t)ru : (int64_t)(ru & ~kCmpTag);
       const uint8_t* src = base + pr * kRowBytes + 16 * (lane ^ (2 * u));
       __builtin_amdgcn_global_load_lds((dec_gbl_void*)src, (dec_lds_void*)(bp + u * 1024), 16, 0, 0);
     }
@@ -512,7 +520,7 @@ __global__ __launch_bounds__(256) void v4_decode_rows_kernel(DecArgs a) {
         const int ruq = __shfl(rz, 16 * j + 8 * q + (lane >> 3), kWave);
         const int u = 8 * q + (lane >> 3);
         const int c = (lane & 7) ^ (2 * ((u >> 2) & 3));
-        const uint8_t* src = a.kv + (int64_t)ruq * kRowBytes + 1024 + 16 * c;
+        const uint8_t* src = (kTails ? a.kv2 + (int64_t)ruq * 128 : a.kv + (int64_t)ruq * kRowBytes + 1024) + 16 * c;
         __builtin_amdgcn_global_load_lds((dec_gbl_void*)src, (dec_lds_void*)(bp + kDecBlk * 1024 + q * 1024), 16, 0, 0);
       }
     }
@@ -805,6 +813,7 @@ static hipError_t dec_launch(int mode, dim3 grid, hipStream_t stream, const DecA
     case 2: return dec_launch_mode<kF16, 2>(grid, stream, a);
     case 3: return dec_launch_mode<kF16, 3>(grid, stream, a);
     case 4: return dec_launch_mode<kF16, 4, 576>(grid, stream, a);
+    case 5: return dec_launch_mode<kF16, 5, 576>(grid, stream, a);
     default: return dec_launch_mode<kF16, 0>(grid, stream, a);
   }
 }
@@ -884,8 +893,12 @@ size_t mla_decode_part_bytes(int64_t T, int64_t H, int64_t topk) {
 }
 
 // Caller: mla_decode_applies(B * S * G, H, topk), H (heads per KV group) % 16 == 0,
-// workspace >= mla_decode_part_bytes.
-hipError_t launch_mla_decode_rows(int is_fp16, const void* q, const void* kv, const int32_t* indices,
+// workspace >= mla_decode_part_bytes.  q_rope / kv_rope: null, or the 64-dim tails of
+// q and kv, which then hold the 512 latent dims alone -- the decode entry's inputs
+// read where they lie (joining them copied the whole pool on every call: 1 row, 128
+// heads, a pool of 6400 rows 37.6 -> 21.7 us).
+hipError_t launch_mla_decode_rows(int is_fp16, const void* q, const void* q_rope, const void* kv, const void* kv_rope,
+                                  const int32_t* indices,
                                   const int32_t* block_table, const int32_t* q_len, const int32_t* kv_len, int64_t B,
                                   int64_t S, int64_t G, int64_t H, int64_t Skv, int64_t block_size,
                                   int64_t max_blocks, int64_t topk, float sm_scale, int causal, void* out, float* lse,
@@ -901,7 +914,9 @@ hipError_t launch_mla_decode_rows(int is_fp16, const void* q, const void* kv, co
   a.mla.block_size = (int)block_size;
   a.mla.max_blocks = (int)max_blocks;
   a.mla.causal = causal;
-  return dec_run(is_fp16, 4, a, q, kv, nullptr, B * S * G, H, topk, nullptr, sm_scale, out, lse, workspace, stream);
+  a.q_rope = static_cast<const uint16_t*>(q_rope);
+  return dec_run(is_fp16, kv_rope ? 5 : 4, a, q, kv, kv_rope, B * S * G, H, topk, nullptr, sm_scale, out, lse,
+                 workspace, stream);
 }
 
 static size_t v4_lists_bytes(int64_t T, int64_t cap) {

@@ -1282,11 +1282,11 @@ size_t mla_workspace_bytes(int64_t tokens, int64_t H, int64_t topk, bool f32) {
 
 bool mla_decode_applies(int64_t T, int64_t H, int64_t topk);
 size_t mla_decode_part_bytes(int64_t T, int64_t H, int64_t topk);
-hipError_t launch_mla_decode_rows(int is_fp16, const void* q, const void* kv, const int32_t* indices,
-                                  const int32_t* block_table, const int32_t* q_len, const int32_t* kv_len, int64_t B,
-                                  int64_t S, int64_t G, int64_t H, int64_t Skv, int64_t block_size,
-                                  int64_t max_blocks, int64_t topk, float sm_scale, int causal, void* out, float* lse,
-                                  void* workspace, hipStream_t stream);
+hipError_t launch_mla_decode_rows(int is_fp16, const void* q, const void* q_rope, const void* kv, const void* kv_rope,
+                                  const int32_t* indices, const int32_t* block_table, const int32_t* q_len,
+                                  const int32_t* kv_len, int64_t B, int64_t S, int64_t G, int64_t H, int64_t Skv,
+                                  int64_t block_size, int64_t max_blocks, int64_t topk, float sm_scale, int causal,
+                                  void* out, float* lse, void* workspace, hipStream_t stream);
 
 // Workspace of launch_sparse_mla: decode rows take the decode kernel's partials.
 size_t sparse_mla_workspace_bytes(int64_t tokens, int64_t H, int64_t topk) {
@@ -1399,8 +1399,8 @@ hipError_t launch_sparse_mla(int is_fp16, const void* q, const void* kv, const i
   if (T == 0 || H == 0) return hipSuccess;
   // Few query rows (decode): the decode kernel, slots across waves and chunks.
   if (mla_decode_applies(T, H, topk))
-    return launch_mla_decode_rows(is_fp16, q, kv, indices, block_table, q_len, kv_len, B, S, G, H, Skv, block_size,
-                                  max_blocks, topk, sm_scale, causal, out, lse, workspace, stream);
+    return launch_mla_decode_rows(is_fp16, q, nullptr, kv, nullptr, indices, block_table, q_len, kv_len, B, S, G, H,
+                                  Skv, block_size, max_blocks, topk, sm_scale, causal, out, lse, workspace, stream);
   MlaArgs a;
   a.q = static_cast<const uint16_t*>(q);
   a.kv = static_cast<const uint16_t*>(kv);
