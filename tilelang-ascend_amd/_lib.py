@@ -6,6 +6,8 @@ not on a HIP device, the call raises -- there is no CPU fallback.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 from pathlib import Path
 from typing import Optional
@@ -111,8 +113,35 @@ def load_library() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
+    _bind_host_path(lib)
     _lib = lib
     return lib
+
+
+HOST_PATH = PKG_DIR / "libdsa_host_path.so"
+_host_path = None
+
+
+def _bind_host_path(lib: ctypes.CDLL) -> None:
+    """Load the wrappers' native host path once and point it at ``lib``'s entry points."""
+    global _host_path
+    if _host_path is None:
+        if not HOST_PATH.exists():
+            raise ImportError(f"{HOST_PATH} is missing: build it with `python tilelang-ascend_amd/build.py`")
+        loader = importlib.machinery.ExtensionFileLoader("dsa_host_path", str(HOST_PATH))
+        spec = importlib.util.spec_from_loader("dsa_host_path", loader)
+        module = importlib.util.module_from_spec(spec)
+        loader.exec_module(module)
+        _host_path = module
+    _host_path.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES})
+
+
+def host_path():
+    """The native host path: each function takes a wrapper's call on plain arguments (exact contiguous
+    tensors on one HIP device, int32 lengths) and returns None where the wrapper must check or convert."""
+    if _host_path is None:
+        load_library()
+    return _host_path
 
 
 TORCH_OPS_PATH = PKG_DIR / "libdsa_torch_ops.so"
@@ -129,6 +158,13 @@ def load_torch_ops():
         torch.ops.load_library(str(TORCH_OPS_PATH))
         _torch_ops_loaded = True
     return torch.ops.dsa
+
+
+def returned(res, what: str):
+    """A host-path result; its return code, when it is one, raises as ``check`` does."""
+    if type(res) is int:
+        check(res, what)
+    return res
 
 
 def check(rc: int, what: str) -> None:

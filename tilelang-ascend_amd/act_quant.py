@@ -26,6 +26,9 @@ def act_quant(x: torch.Tensor, round_scale: bool = False,
               dtype: torch.dtype = torch.int8) -> Tuple[torch.Tensor, torch.Tensor]:
     """(y, scales): y has x's shape in ``dtype``; scales [M, 1] fp32 for a 2-D x
     ([B, S, 1] for a 3-D one, as act_quant.py:138-140 returns them)."""
+    res = _lib.host_path().act_quant(x, round_scale, _OUT.get(dtype))
+    if res is not None:
+        return _lib.returned(res, "dsa_act_quant")
     if x.dtype not in _IN:
         raise ValueError(f"x must be bfloat16, float16 or float32, got {x.dtype}")
     if dtype not in _OUT:

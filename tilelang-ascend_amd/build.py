@@ -22,6 +22,8 @@ LIB_PATH = PKG_DIR / LIB_NAME
 # torch.ops.dsa.* registrations (csrc/torch_ops.cpp): host C++ over the C ABI, linked against
 # libdsa_mi355x.so and libtorch; built separately so the C-ABI library stays free of torch.
 TORCH_OPS_PATH = PKG_DIR / "libdsa_torch_ops.so"
+# The wrappers' native host path (csrc/host_path.cpp): a Python extension module over the C ABI.
+HOST_PATH = PKG_DIR / "libdsa_host_path.so"
 ARCH = "gfx950"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -75,7 +77,9 @@ def build(verbose: bool = False, jobs: int = 8) -> Path:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
-    build_torch_ops(verbose)
+    with cf.ThreadPoolExecutor(max_workers=2) as ex:
+        for f in [ex.submit(build_torch_ops, verbose), ex.submit(build_host_path, verbose)]:
+            f.result()
     return LIB_PATH
 
 
@@ -99,6 +103,30 @@ def build_torch_ops(verbose: bool = False) -> Path:
         raise RuntimeError(f"torch_ops.cpp failed:\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, TORCH_OPS_PATH)
     return TORCH_OPS_PATH
+
+
+def build_host_path(verbose: bool = False) -> Path:
+    """Compile csrc/host_path.cpp (host only, g++) into libdsa_host_path.so."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    torch_lib = Path(torch.__file__).resolve().parent / "lib"
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={abi}", "-DUSE_ROCM",
+           "-D__HIP_PLATFORM_AMD__", *[f"-I{d}" for d in cpp_extension.include_paths()], "-I/opt/rocm/include",
+           f"-I{sysconfig.get_paths()['include']}", str(CSRC / "host_path.cpp"), "-o", str(tmp), f"-L{torch_lib}",
+           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
+           f"-Wl,-rpath,{torch_lib}"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"host_path.cpp failed:\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, HOST_PATH)
+    return HOST_PATH
 
 
 if __name__ == "__main__":

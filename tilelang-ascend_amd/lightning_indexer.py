@@ -30,6 +30,9 @@ _KINDS = {
 }
 
 
+_NATIVE_LAYOUTS = {("BSND", "BSND"), ("BSND", "PA_BSND"), ("TND", "TND"), ("TND", "PA_BSND")}
+
+
 def _per_batch(seq_len: Optional[torch.Tensor], B: int, default: int, device) -> Optional[torch.Tensor]:
     if seq_len is None:
         return None
@@ -248,6 +251,14 @@ def lightning_indexer(query: torch.Tensor, key: torch.Tensor, weights: torch.Ten
     bit.  The default (None) streams calls of at least 2048 rows longer than 32768 keys, where it
     is faster.
     """
+    if (not tuning and query_scale is None and pre_tokens == next_tokens == _INT64_MAX
+            and (layout_query, layout_key) in _NATIVE_LAYOUTS
+            and (block_table is None) == (layout_key != "PA_BSND")):
+        res = _lib.host_path().indexer(query, key, weights, actual_seq_lengths_query, actual_seq_lengths_key,
+                                       block_table, layout_query == "TND", sparse_count, sparse_mode, return_value,
+                                       key_scale, fuse_topk)
+        if res is not None:
+            return _lib.returned(res, "dsa_lightning_indexer")
     unknown = set(tuning) - {"block_n", "pp_slots", "max_cores"}
     if unknown:
         raise TypeError(f"unexpected keyword arguments {sorted(unknown)}")

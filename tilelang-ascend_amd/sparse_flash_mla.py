@@ -68,6 +68,13 @@ def sparse_flash_mla(
     reference's asserts raise ``AssertionError`` here too).
     """
     del seqused_q, core_num
+    if (layout_q == "TND" and ori_mask_mode == 4 and (cmp_mask_mode == 3 or cmp_kv is None) and ori_win_right == 0
+            and layout_kv == "PA_ND" and topk_cmp is None):
+        res = _lib.host_path().flash_mla(q, ori_kv, cmp_kv, cmp_sparse_indices, ori_block_table, cmp_block_table,
+                                         cu_seqlens_q, seqused_kv, sinks, softmax_scale, cmp_ratio, ori_win_left,
+                                         return_softmax_lse)
+        if res is not None:
+            return _lib.returned(res, "dsa_sparse_flash_mla")
     if ori_mask_mode != 4:
         raise AssertionError("only ori_mask_mode=4 supported")
     if not (cmp_mask_mode == 3 or cmp_kv is None):

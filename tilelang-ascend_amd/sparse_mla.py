@@ -52,6 +52,10 @@ def sparse_mla_fwd(q: torch.Tensor, kv: torch.Tensor, indices: torch.Tensor, sm_
                    actual_seq_lengths_kv: Optional[torch.Tensor] = None,
                    is_causal: bool = True) -> Tuple[torch.Tensor, torch.Tensor]:
     """Sparse MLA forward; returns ``(out [B, S, H, 512], lse [B, S, H] fp32)``."""
+    res = _lib.host_path().sparse_mla(q, kv, indices, D_QK ** -0.5 if sm_scale is None else sm_scale, block_table,
+                                      actual_seq_lengths_query, actual_seq_lengths_kv, is_causal)
+    if res is not None:
+        return _lib.returned(res, "dsa_sparse_mla_fwd")
     if q.dtype not in _KINDS:
         raise ValueError(f"q must be bfloat16 or float16, got {q.dtype}")
     if kv.dtype != q.dtype:
@@ -132,6 +136,10 @@ def sparse_gqa_fwd(q: torch.Tensor, kv: torch.Tensor, indices: torch.Tensor, sm_
     (g+1)*H/G - 1 read KV head g.  sm_scale defaults to 128^-0.5; slot validity,
     causality and lengths as ``sparse_mla_fwd``.
     """
+    res = _lib.host_path().sparse_gqa(q, kv, indices, D_GQA ** -0.5 if sm_scale is None else sm_scale,
+                                      actual_seq_lengths_query, actual_seq_lengths_kv, is_causal)
+    if res is not None:
+        return _lib.returned(res, "dsa_sparse_attention_fwd")
     if q.dtype not in _KINDS:
         raise ValueError(f"q must be bfloat16 or float16, got {q.dtype}")
     if kv.dtype != q.dtype:
@@ -232,10 +240,12 @@ def sparse_attn_tilelang(query, key, value, sparse_indices, scale_value, sparse_
     del value, sparse_block_size, layout_query, layout_kv, attention_mode
     if query_rope is None or key_rope is None:
         raise ValueError("query_rope and key_rope are required (D = 512 + 64)")
-    out = _decode_parts(query, key, query_rope, key_rope, sparse_indices, scale_value, actual_seq_lengths_query,
-                        actual_seq_lengths_kv, sparse_mode, block_table)
+    # The parts as they lie, where the decode kernel takes them: up to 8 rows of plain tensors.  The
+    # rest (other layouts, mixed dtypes, parts off 16 bytes) is joined, and checked or refused joined.
+    out = _lib.host_path().decode_parts(query, key, query_rope, key_rope, sparse_indices, scale_value,
+                                        actual_seq_lengths_query, actual_seq_lengths_kv, sparse_mode == 3, block_table)
     if out is not None:
-        return out
+        return _lib.returned(out, "dsa_sparse_mla_decode_parts")
     q = torch.cat((query.unsqueeze(0), query_rope.unsqueeze(0)), dim=-1).contiguous()
     kv = torch.cat((key, key_rope), dim=-1).contiguous()
     T = q.shape[1]
@@ -244,53 +254,3 @@ def sparse_attn_tilelang(query, key, value, sparse_indices, scale_value, sparse_
                             actual_seq_lengths_query=actual_seq_lengths_query,
                             actual_seq_lengths_kv=actual_seq_lengths_kv, is_causal=sparse_mode == 3)
     return out.squeeze(0)
-
-
-
-def _decode_parts(query, key, query_rope, key_rope, sparse_indices, scale_value, q_lens, kv_lens, sparse_mode,
-                  block_table):
-    """``sparse_attn_tilelang`` on the parts as they lie, or None where they must be joined: more than
-    8 rows, or parts of other shapes, mixed dtypes, not contiguous or off 16 bytes (joining and the
-    joined call's own checks take or refuse those)."""
-    parts = (query, query_rope, key, key_rope)
-    if query.dim() != 3 or key.dim() != 4 or query.shape[2] != D_V or not query.is_cuda:
-        return None
-    T, N, _ = query.shape
-    rope = D_QK - D_V
-    if query_rope.shape != (T, N, rope) or key.shape[2:] != (1, D_V) or key_rope.shape != key.shape[:3] + (rope,):
-        return None
-    dt, dev = query.dtype, query.device
-    for t in parts:
-        if t.dtype != dt or t.device != dev or not t.is_contiguous() or t.data_ptr() & 15:
-            return None
-    topk = sparse_indices.numel() // T if T else 0
-    lib = _lib.load_library()
-    if dt not in _KINDS or not lib.dsa_sparse_mla_decode_parts_applies(1, T, N, topk):
-        return None
-    if not sparse_indices.is_cuda or sparse_indices.device != dev or topk * T != sparse_indices.numel():
-        return None
-    if block_table is None:
-        if key.shape[0] != 1:
-            return None
-        bt, block_size, max_blocks, skv = None, 0, 0, key.shape[1]
-    else:
-        bt = block_table.to(torch.int32).contiguous()
-        if bt.dim() != 2 or bt.shape[0] != 1 or bt.device != dev:
-            return None
-        block_size, max_blocks = key.shape[1], bt.shape[1]
-        skv = max_blocks * block_size
-    idx = sparse_indices.to(torch.int32).contiguous()
-    ql = _lens(q_lens, 1, dev)
-    kl = _lens(kv_lens, 1, dev)
-    out = torch.empty((T, N, D_V), dtype=dt, device=dev)
-    ws_bytes = lib.dsa_sparse_mla_workspace_size(1, T, N, topk)
-    # One allocation for the LSE and the workspace.
-    scratch = torch.empty((T * N * 4 + 256 + ws_bytes,), dtype=torch.uint8, device=dev)
-    lse = scratch.data_ptr()
-    rc = lib.dsa_sparse_mla_decode_parts(_KINDS[dt], query.data_ptr(), query_rope.data_ptr(), key.data_ptr(),
-                                         key_rope.data_ptr(), idx.data_ptr(), _lib.ptr(bt), _lib.ptr(ql), _lib.ptr(kl),
-                                         1, T, N, skv, block_size, max_blocks, topk, float(scale_value),
-                                         1 if sparse_mode == 3 else 0, out.data_ptr(), lse,
-                                         lse + (T * N * 4 + 255) // 256 * 256, ws_bytes, _lib.stream_handle(dev))
-    _lib.check(rc, "dsa_sparse_mla_decode_parts")
-    return out

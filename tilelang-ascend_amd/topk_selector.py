@@ -24,6 +24,9 @@ def topk_selector(x: torch.Tensor, top_k: int, sorted: bool = True, *, row_len: 
     ``row_len`` (int32, one per row) excludes columns >= row_len[r].
     fp16/bf16 inputs are widened to fp32 on the device (exact).
     """
+    res = _lib.host_path().topk(x, top_k, sorted, row_len, return_values)
+    if res is not None:
+        return _lib.returned(res, "dsa_topk_select_ws")
     if x.dim() < 1:
         raise ValueError("x must have at least one dimension")
     if not (1 <= top_k <= 8192):
