@@ -275,3 +275,26 @@ def test_decode_parts_equal_the_joined_call(dsa, dev, T, N, topk, nb, dtype):
         same = dsa.sparse_attn_tilelang(qt, k, k, idx.view(T, 1, topk), 0.05, 1, ql, kl, query_rope=qr, key_rope=kr,
                                         sparse_mode=mode, block_table=bt)
         assert torch.equal(out, same)
+
+
+@pytest.mark.parametrize("h", [32, 48, 64, 80])
+@pytest.mark.parametrize("topk", [1, 31, 33, 200, 2080])
+def test_row_lists_head_and_tile_edges(dsa, dev, h, topk):
+    """More than 8 rows, so the row-list kernels: both sides of their head counts (one wave, four waves
+    of 16 heads with a missing and with every block, four of 32) by list lengths of less than a tile, a
+    tile and one row, many tiles, and more slots than one workgroup holds (split partials); -1 slots
+    leave the first, a middle or every tile of some rows empty.  Bars as the module's bf16 ones."""
+    g = torch.Generator().manual_seed(h + topk)
+    m, n = 10, 2200
+    q = (torch.randn(1, m, h, 512, generator=g) * 0.5).to(torch.bfloat16)
+    kv = (torch.randn(1, n, 512, generator=g) * 0.5).to(torch.bfloat16)
+    idx = torch.stack([torch.randperm(n, generator=g)[:topk] for _ in range(m)]).to(torch.int32).view(1, m, topk)
+    idx[0, 1, :32] = -1
+    idx[0, 2, 32:96] = -1
+    idx[0, 3] = -1
+    sink = torch.randn(h, generator=g)
+    scale = 512 ** -0.5
+    out = _run(dsa, dev, q, kv, sink, idx, scale)
+    want, want_lse = ref.sparse_attn_sink(q, kv, sink, idx, scale)
+    torch.testing.assert_close(out, want, atol=4e-3, rtol=2e-3)
+    torch.testing.assert_close(_lse(dsa, dev, q, kv, sink, idx, scale), want_lse, rtol=1e-3, atol=1e-3)

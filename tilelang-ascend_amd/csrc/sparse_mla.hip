@@ -43,10 +43,10 @@
 // into slices between them.  With more than one split a workgroup writes a
 // normalised bf16 partial and its LSE; a combine kernel merges them.
 //
-// The 512-wide row lists of up to 64 heads (one or two waves) run the same
-// body from a two-stage ring instead (sparse_mla_rows2_kernel): one tile is
-// computed at a time while the next arrives, in 73 KB of LDS, so that two
-// workgroups share a CU and every SIMD holds a wave.
+// The 512-wide row lists of up to 32 heads (one wave) run the same body from a
+// two-stage ring instead (sparse_mla_rows2_kernel): one tile is computed at a
+// time while the next arrives, in 73 KB of LDS, so that two workgroups share a
+// CU.  Those of 33 to 64 heads have a kernel of their own (sparse_mla_rows4_kernel).
 #include "common.hpp"
 
 namespace dsa {
@@ -617,11 +617,11 @@ __device__ __attribute__((noinline)) void mla_exact_fallback(const uint16_t* q, 
 
 // kPaged: the KV rows are addressed through a block table (a.block_table).
 // kSt: ring stages.  4 (sparse_mla_kernel): the pipelined loop below.  2
-// (sparse_mla_rows2_kernel: the 512-wide row lists with one or two waves, i.e. up
-// to 64 heads): each tile is computed in turn -- Q K^T, softmax, P V -- while the
+// (sparse_mla_rows2_kernel: the 512-wide row lists with one wave, i.e. up to 32
+// heads): each tile is computed in turn -- Q K^T, softmax, P V -- while the
 // next tile's DMA fills the other stage; the 73 KB of LDS let two workgroups
-// share a CU, so all four SIMDs work and each workgroup's exposed DMA latency,
-// prologue and epilogue overlap the other's.
+// share a CU, and each workgroup's exposed DMA latency, prologue and epilogue
+// overlap the other's.
 template <int kNW, bool kF16, int kD, bool kPaged, int kSt>
 __device__ __forceinline__ void sparse_mla_body(MlaArgs a) {
   static_assert(kSt == kStages || kSt == 2, "ring stages");
@@ -1123,9 +1123,324 @@ __global__ __launch_bounds__(kNW * kWave) void sparse_mla_kernel(MlaArgs a) {
   sparse_mla_body<kNW, kF16, kD, kPaged, kStages>(a);
 }
 
-template <int kNW, bool kF16>
-__global__ __launch_bounds__(kNW * kWave) void sparse_mla_rows2_kernel(MlaArgs a) {
-  sparse_mla_body<kNW, kF16, 512, false, 2>(a);
+template <bool kF16>
+__global__ __launch_bounds__(kWave) void sparse_mla_rows2_kernel(MlaArgs a) {
+  sparse_mla_body<1, kF16, 512, false, 2>(a);
+}
+
+// ---------------------------------------------------------------------------
+// The 512-wide row lists of 33 to 64 heads: four waves of 16 heads, two waves
+// per SIMD.  A tile is computed in turn -- Q K^T, softmax, P V -- from a
+// two-stage ring while the next tile's DMA fills the other stage, and nothing
+// inside a wave overlaps these; a second wave on its SIMD (the workgroup has a
+// neighbour on the CU: 78 KB of LDS, 256 registers a wave) does.  That fits
+// because P V is split by output columns: wave w holds O for all 64 heads and
+// columns 128 w .. (128 registers instead of the 256 of 32 heads x 512 columns),
+// reads each V operand once per workgroup, and gets the other waves' P (16 heads
+// x 32 keys a wave) through LDS.  Against one wave per SIMD of 32 heads each, 8192
+// rows by 64 heads, row lists included: window + 512 selected rows 783 -> 666 us,
+// window alone 359 -> 294, window + 64 dense rows 414 -> 347 (outputs bit-equal).
+constexpr int kR4Waves = 4;
+constexpr int kR4Heads = 64;                            // heads per workgroup
+constexpr int kR4PBytes = kR4Waves * 1024;              // one P operand per wave
+constexpr int kR4POffset = MlaLayout<512, 2>::kLds;
+constexpr int kR4Lds = kR4POffset + kR4PBytes;
+static_assert(2 * kR4Lds <= 160 * 1024, "two workgroups per CU");
+// K operands in flight: 1 takes 723 us where 2 and 3 take 699 and 712 (the second
+// wave hides the rest), 4 no longer fits the registers (950).
+constexpr int kR4Ahead = 2;
+
+__device__ __forceinline__ void r4_p_write(const u32x4& p, uint32_t addr) {
+  __asm__ __volatile__("ds_write_b128 %0, %1" ::"v"(addr), "v"(p) : "memory");
+}
+
+template <int J>
+__device__ __forceinline__ void r4_k_read(u32x4 (&k)[kR4Ahead + 1], const uint32_t (&qa)[2]) {
+  b128_read<4096 * (J / 4) + 2048 * (J % 2)>(k[J % (kR4Ahead + 1)], qa[(J / 2) % 2]);
+}
+template <int J = 0>
+__device__ __forceinline__ void r4_k_first(u32x4 (&k)[kR4Ahead + 1], const uint32_t (&qa)[2]) {
+  if constexpr (J < kR4Ahead) {
+    r4_k_read<J>(k, qa);
+    r4_k_first<J + 1>(k, qa);
+  }
+}
+// Half-step J of S^T = K Q^T: key half J % 2 of dim step J / 2, accumulator sets
+// by the parity of the step (the sums of qk_half).
+template <bool kF16, bool kDma, int J>
+__device__ __forceinline__ void r4_qk(f32x4 (&c)[2][2], const u32x4 (&qb)[16], const uint32_t (&qa)[2],
+                                      u32x4 (&k)[kR4Ahead + 1], TileDma<kR4Waves, 512>& dma) {
+  constexpr int kHalf = MlaGeom<512>::kQkHalf;
+  if constexpr (J + kR4Ahead < kHalf) r4_k_read<J + kR4Ahead>(k, qa);
+  if constexpr (kDma) il_dma<kR4Waves, 512, J>(dma);
+  constexpr int kWait = (kHalf - 1 - J) < kR4Ahead ? (kHalf - 1 - J) : kR4Ahead;
+  u32x4& kj = k[J % (kR4Ahead + 1)];
+  lgkm_wait_k<kWait>(kj);
+  mfma_qk<kF16, (J < 4)>(c[(J / 2) % 2][J % 2], kj, qb[J / 2]);
+  if constexpr (J + 1 < kHalf) r4_qk<kF16, kDma, J + 1>(c, qb, qa, k, dma);
+}
+
+// V group kG (two 16-column blocks) times head block kB of the wave's order (0: its own).
+template <bool kF16, int kG, int kB>
+__device__ __forceinline__ void r4_pv(f32x4 (&o)[4][8], const u32x2 (&v)[4], const u32x4& p) {
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const u32x4 vb = {v[2 * j].x, v[2 * j].y, v[2 * j + 1].x, v[2 * j + 1].y};
+    o[kB][2 * kG + j] = mfma16<kF16>(vb, p, o[kB][2 * kG + j]);
+  }
+}
+template <bool kF16, int kG>
+__device__ __forceinline__ void r4_pv_group(f32x4 (&o)[4][8], u32x2 (&v)[2][4], const uint32_t (&va)[2], const u32x4& pa,
+                                            const u32x4 (&px)[3]) {
+  if constexpr (kG < 3) pv_group_reads<kG + 1>(v[(kG + 1) % 2], va);
+  lgkm_wait<(kG < 3 ? 4 : 0)>(v[kG % 2]);
+  r4_pv<kF16, kG, 0>(o, v[kG % 2], pa);
+  r4_pv<kF16, kG, 1>(o, v[kG % 2], px[0]);
+  r4_pv<kF16, kG, 2>(o, v[kG % 2], px[1]);
+  r4_pv<kF16, kG, 3>(o, v[kG % 2], px[2]);
+}
+
+template <bool kF16>
+__global__ __launch_bounds__(kR4Waves * kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void sparse_mla_rows4_kernel(MlaArgs a) {
+  using Lay = MlaLayout<512, 2>;
+  constexpr int kStageBytes = MlaGeom<512>::kStageBytes;
+  constexpr int kThreads = kR4Waves * kWave;
+  extern __shared__ __align__(128) uint8_t lds[];
+  int32_t* rows = reinterpret_cast<int32_t*>(lds + Lay::kRowsOffset);
+  uint32_t* tile_mask = reinterpret_cast<uint32_t*>(lds + Lay::kTileMaskOffset);
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int r = lane & 15;
+  const int g = lane >> 4;
+  const int T = a.B * a.S;
+  const int token = blockIdx.x % T;
+  const int split = blockIdx.x / T;
+  const int group0 = blockIdx.y * kR4Heads;
+  const int head0 = group0 + 16 * wave;  // this wave's Q K^T heads; past H they repeat head H - 1, unstored
+
+  // Slots first, then Q (as in sparse_mla_body): every load from a clamped valid address.
+  const int32_t* irow = a.indices + (int64_t)token * a.topk;
+  const int slot_begin = split * a.keys_per_split;
+  const int count_raw = a.slot_count[token];  // negative: a padded query row (out = 0, lse = 0)
+  const int row_slots = min(max(count_raw, 0), a.topk);
+  const int slot_end = min(row_slots, slot_begin + a.keys_per_split);
+  const int nslots = max(slot_end - slot_begin, 0);
+  constexpr int kIdxPerLane = kSlotsCap / kThreads;
+  const int last_slot = max(min(slot_end, a.topk) - 1, 0);
+  int idx_raw[kIdxPerLane];
+#pragma unroll
+  for (int j = 0; j < kIdxPerLane; ++j) idx_raw[j] = irow[min(slot_begin + tid + j * kThreads, last_slot)];
+  __asm__ __volatile__("" ::: "memory");
+  u32x4 qb[16];
+  {
+    const uint16_t* qp = a.q + ((int64_t)token * a.H + min(head0 + r, a.H - 1)) * 512 + 8 * g;
+#pragma unroll
+    for (int st = 0; st < 16; ++st) qb[st] = *reinterpret_cast<const u32x4*>(qp + 32 * st);
+  }
+  const bool row_active = count_raw >= 0;
+  int ntiles = row_active ? (nslots + kMlaTile - 1) / kMlaTile : 0;
+  int32_t* first_valid = rows + kSlotsCap + 1;
+  int32_t* last_valid = rows + kSlotsCap + 2;
+  if (tid == 0) {
+    *first_valid = 0x7fffffff;
+    *last_valid = -1;
+  }
+  __syncthreads();
+  int wave_first = 0x7fffffff, wave_last = -1;
+#pragma unroll
+  for (int j = 0; j < kIdxPerLane; ++j) {
+    const int i0 = wave * kWave + j * kThreads;
+    const int i = i0 + lane;
+    const int row = row_active && i < nslots && idx_raw[j] >= 0 ? idx_raw[j] : -1;
+    if (i < ntiles * kMlaTile) rows[i] = row;
+    const uint64_t vm = __ballot(row >= 0 && i < ntiles * kMlaTile);
+    if (vm != 0) {
+      wave_first = min(wave_first, i0 + (int)__builtin_ctzll(vm));
+      wave_last = max(wave_last, i0 + 63 - (int)__builtin_clzll(vm));
+    }
+    if (lane == 0 && i0 < ntiles * kMlaTile) {
+      tile_mask[i0 / kMlaTile] = (uint32_t)vm;
+      if (i0 / kMlaTile + 1 < ntiles) tile_mask[i0 / kMlaTile + 1] = (uint32_t)(vm >> 32);
+    }
+  }
+  if (lane == 0 && wave_first != 0x7fffffff) {
+    atomicMin(first_valid, wave_first);
+    atomicMax(last_valid, wave_last);
+  }
+  __syncthreads();
+  // Leading and trailing tiles without a valid slot are skipped; the first valid
+  // slot's row stands in for empty ones (sparse_mla_body).
+  const int fv = *first_valid;
+  const int safe_row = fv < kSlotsCap ? rows[fv] : -1;
+  const int nslots_all = ntiles * kMlaTile;
+  const int t_first = safe_row < 0 ? 0 : fv / kMlaTile;
+  ntiles = safe_row < 0 ? 0 : min(ntiles, *last_valid / kMlaTile + 1) - t_first;
+  const int32_t* trows = rows + t_first * kMlaTile;
+  const uint32_t* tmask = tile_mask + t_first;
+  const uint8_t* kvb = reinterpret_cast<const uint8_t*>(a.kv);
+  const uint8_t* kvb2 = reinterpret_cast<const uint8_t*>(a.kv2);
+
+  f32x4 o[4][8];
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_ref = -__builtin_huge_valf(), lsum = 0.f, lsum_r = 0.f;
+  bool overflow = false;
+  const float scale_log2 = a.scale_log2;
+  // Operand addresses in a stage (sparse_mla_body); odd steps and column pairs differ in bit 6 alone.
+  const uint32_t qk_lane = 1024 * (r >> 3) + 128 * (r & 7) + 16 * (g ^ lds_swizzle(r & 7, r >> 3));
+  const int pv_u = 4 * (g & 1) + (r >> 2);
+  const uint32_t pv_lane = 1024 * (g >> 1) + 128 * pv_u + 16 * ((r & 3) ^ lds_swizzle(pv_u, g >> 1)) + 8192 * wave;
+  const uint32_t p_base = lds_u32(lds + kR4POffset) + 16 * lane;
+
+  if (ntiles > 0) {
+    TileDma<kR4Waves, 512> dma;
+    dma.prepare(kvb, kvb2, trows, safe_row, 0, lds, wave, lane);
+    il_dma_all(dma);
+  }
+  for (int tile = 0; tile < ntiles; ++tile) {
+    // The tile has arrived (so has Q); the barrier publishes it and certifies
+    // that every wave is done with the last tile and its P.
+    wait_vmcnt<0>();
+    raw_barrier();
+    const bool more = tile + 1 < ntiles;  // workgroup-uniform
+    TileDma<kR4Waves, 512> dma;
+    if (more) dma.prepare(kvb, kvb2, trows, safe_row, tile + 1, lds + ((tile + 1) & 1) * kStageBytes, wave, lane);
+    const uint32_t mask = __builtin_amdgcn_readfirstlane(tmask[tile]);
+    const uint32_t base = lds_u32(lds + (tile & 1) * kStageBytes);
+    const uint32_t qa[2] = {base + qk_lane, (base + qk_lane) ^ 64};
+    const uint32_t va[2] = {base + pv_lane, (base + pv_lane) ^ 64};
+    f32x4 c[2][2];
+    u32x4 k[kR4Ahead + 1];
+    r4_k_first(k, qa);
+    if (more) r4_qk<kF16, true, 0>(c, qb, qa, k, dma);
+    else r4_qk<kF16, false, 0>(c, qb, qa, k, dma);
+    static_assert(kR4Ahead + 1 == 3, "the wait below names every K operand register");
+    // 24 wait states between the asm MFMAs and the first VALU read of a score (qk_phase).
+    __asm__ __volatile__("s_nop 7\n\ts_nop 7\n\ts_nop 7"
+                         : "+v"(c[0][0]), "+v"(c[0][1]), "+v"(c[1][0]), "+v"(c[1][1]), "+v"(k[0]), "+v"(k[1]),
+                           "+v"(k[2]));
+    float s[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s[e] = c[0][e / 4][e % 4] + c[1][e / 4][e % 4];
+    if (mask != 0xffffffffu) {
+      const uint32_t bits = ((mask >> (4 * g)) & 15u) | (((mask >> (16 + 4 * g)) & 15u) << 4);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s[e] = ((bits >> e) & 1u) ? s[e] : -__builtin_huge_valf();
+    }
+    if (tile == 0) {  // holds the first valid slot: fixes the reference
+      float cmax = s[0];
+#pragma unroll
+      for (int e = 1; e < 8; ++e) cmax = fmaxf(cmax, s[e]);
+      cmax = fmaxf(cmax, __shfl_xor(cmax, 16, kWave));
+      cmax = fmaxf(cmax, __shfl_xor(cmax, 32, kWave));
+      m_ref = cmax * scale_log2 + PRange<kF16>::kRefBias;
+    }
+    const float neg_m = -m_ref;
+    float p[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) p[e] = fast_exp2(fmaf(s[e], scale_log2, neg_m));
+    const float ps = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+    lsum += ps;
+    overflow = overflow || !(ps <= kOverflowSumOf<kF16>);
+    const u32x4 pa = {pack2<kF16>(p[0], p[1]), pack2<kF16>(p[2], p[3]), pack2<kF16>(p[4], p[5]),
+                      pack2<kF16>(p[6], p[7])};
+    r4_p_write(pa, p_base + 1024 * wave);
+    u32x2 v[2][4];
+    pv_group_reads<0>(v[0], va);
+    lsum_r += ((unpack_lo<kF16>(pa.x) + unpack_hi<kF16>(pa.x)) + (unpack_lo<kF16>(pa.y) + unpack_hi<kF16>(pa.y))) +
+              ((unpack_lo<kF16>(pa.z) + unpack_hi<kF16>(pa.z)) + (unpack_lo<kF16>(pa.w) + unpack_hi<kF16>(pa.w)));
+    lgkm_wait<0>(v[0]);  // P is written too
+    raw_barrier();
+    u32x4 px[3];
+    b128_read<0>(px[0], p_base + 1024 * ((wave + 1) & 3));
+    b128_read<0>(px[1], p_base + 1024 * ((wave + 2) & 3));
+    b128_read<0>(px[2], p_base + 1024 * ((wave + 3) & 3));
+    pv_group_reads<1>(v[1], va);
+    r4_pv<kF16, 0, 0>(o, v[0], pa);
+    lgkm_wait_k<6>(px[0]);
+    r4_pv<kF16, 0, 1>(o, v[0], px[0]);
+    lgkm_wait_k<5>(px[1]);
+    r4_pv<kF16, 0, 2>(o, v[0], px[1]);
+    lgkm_wait_k<4>(px[2]);
+    r4_pv<kF16, 0, 3>(o, v[0], px[2]);
+    r4_pv_group<kF16, 1>(o, v, va, pa, px);
+    r4_pv_group<kF16, 2>(o, v, va, pa, px);
+    r4_pv_group<kF16, 3>(o, v, va, pa, px);
+  }
+  // All LDS reads and DMAs retire before the ring is reused below.
+  __builtin_amdgcn_s_waitcnt(0);
+  int32_t* overflow_flag = rows + kSlotsCap;
+  if (tid == 0) *overflow_flag = 0;
+  __syncthreads();
+  if (__any(overflow) && lane == 0) *overflow_flag = 1;
+  __syncthreads();
+  const bool final_out = a.splits == 1;
+  uint16_t* obase = final_out ? a.out : a.part_o + (int64_t)split * T * a.H * kMlaDV;
+  float* obase32 = nullptr;
+  if (a.out32) obase32 = final_out ? a.out32 : a.part_o32 + (int64_t)split * T * a.H * kMlaDV;
+  float* lbase = final_out ? a.lse : a.part_lse + (int64_t)split * T * a.H;
+  const float* sinks = final_out ? a.sinks : nullptr;  // else they join in the combine
+  if (*overflow_flag) {
+    mla_exact_fallback<kF16, 512>(a.q, kvb, kvb2, sinks, obase, obase32, lbase, a.H, scale_log2, rows, nslots_all, token,
+                                  group0, kR4Heads, reinterpret_cast<float*>(lds), kThreads);
+    return;
+  }
+  // Normalisers of this wave's heads (sparse_mla_body's: O by the rounded weights,
+  // the LSE by the exact sum, the sink in both), then round to every wave.
+  {
+    float l_tot = lsum, l_r = lsum_r;
+    l_tot += __shfl_xor(l_tot, 16, kWave);
+    l_tot += __shfl_xor(l_tot, 32, kWave);
+    l_r += __shfl_xor(l_r, 16, kWave);
+    l_r += __shfl_xor(l_r, 32, kWave);
+    float inv = l_r > 0.f ? 1.f / l_r : 0.f, m_out = m_ref;
+    const int h = head0 + r;
+    if (sinks) {
+      const float sink = sinks[min(h, a.H - 1)] * 1.4426950408889634f;
+      const float mm = fmaxf(m_ref, sink);
+      const float so = fast_exp2(m_ref - mm);
+      const float es = fast_exp2(sink - mm);
+      l_tot = l_tot * so + es;
+      inv = so / (l_r * so + es);
+      m_out = mm;
+    }
+    if (!row_active) {
+      inv = 0.f;
+      l_tot = 1.f;
+      m_out = 0.f;
+    }
+    if (g == 0) {
+      reinterpret_cast<float*>(lds)[16 * wave + r] = inv;
+      if (h < a.H)
+        lbase[(int64_t)token * a.H + h] =
+            l_tot > 0.f ? (m_out + fast_log2(l_tot)) * 0.69314718055994531f : -__builtin_huge_valf();
+    }
+  }
+  __syncthreads();
+  // Lane (g, r) of block b holds head r's columns 32 p2 + 8 g .. + 7 of the wave's 128.
+  const int col0 = 128 * wave + 8 * g;
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const int hb = 16 * ((wave + b) & 3);
+    const float inv = reinterpret_cast<const float*>(lds)[hb + r];
+    if (group0 + hb >= a.H) continue;  // wave-uniform
+    const int64_t orow = ((int64_t)token * a.H + group0 + hb + r) * kMlaDV + col0;
+#pragma unroll
+    for (int p2 = 0; p2 < 4; ++p2) {
+      const f32x4 x = o[b][2 * p2] * inv, y = o[b][2 * p2 + 1] * inv;
+      if (obase32) {
+        *reinterpret_cast<f32x4*>(obase32 + orow + 32 * p2) = x;
+        *reinterpret_cast<f32x4*>(obase32 + orow + 32 * p2 + 4) = y;
+      } else {
+        *reinterpret_cast<u32x4*>(obase + orow + 32 * p2) =
+            u32x4{pack2<kF16>(x[0], x[1]), pack2<kF16>(x[2], x[3]), pack2<kF16>(y[0], y[1]), pack2<kF16>(y[2], y[3])};
+      }
+    }
+  }
 }
 
 // Merge split partials: lse = log(sum_i exp(lse_i) [+ exp(sink)]),
@@ -1326,12 +1641,16 @@ hipError_t mla_scratch_ptr(void** out) {
 template <int kNW, bool kF16, int kD, bool kPaged>
 static hipError_t launch_mla_kernel(const MlaArgs& a, int head_groups, hipStream_t stream) {
   const dim3 grid((unsigned)((int64_t)a.B * a.S * a.G * a.splits), (unsigned)head_groups);
-  if constexpr (kD == 512 && kNW <= 2) {
-    // Two-stage ring for the 512-wide row lists of up to 64 heads (see the kernel).
-    constexpr int kLds = MlaLayout<512, 2>::kLds;
-    const hipError_t ea = set_dynamic_lds_once<sparse_mla_rows2_kernel<kNW, kF16>>(kLds);
+  if constexpr (kD == 512 && kNW == 2) {
+    const hipError_t ea = set_dynamic_lds_once<sparse_mla_rows4_kernel<kF16>>(kR4Lds);
     if (ea != hipSuccess) return ea;
-    hipLaunchKernelGGL((sparse_mla_rows2_kernel<kNW, kF16>), grid, dim3(kNW * kWave), kLds, stream, a);
+    hipLaunchKernelGGL((sparse_mla_rows4_kernel<kF16>), grid, dim3(kR4Waves * kWave), kR4Lds, stream, a);
+  } else if constexpr (kD == 512 && kNW == 1) {
+    // Two-stage ring for the 512-wide row lists of up to 32 heads (see the kernel).
+    constexpr int kLds = MlaLayout<512, 2>::kLds;
+    const hipError_t ea = set_dynamic_lds_once<sparse_mla_rows2_kernel<kF16>>(kLds);
+    if (ea != hipSuccess) return ea;
+    hipLaunchKernelGGL((sparse_mla_rows2_kernel<kF16>), grid, dim3(kWave), kLds, stream, a);
   } else {
     constexpr int kLds = MlaLayout<kD, kStages>::kLds;
     const hipError_t ea = set_dynamic_lds_once<sparse_mla_kernel<kNW, kF16, kD, kPaged>>(kLds);
