@@ -182,3 +182,37 @@ def test_large_score_jumps(dsa, dev, jump, S):
     assert torch.isfinite(out.float()).all() and torch.isfinite(lse).all()
     torch.testing.assert_close(out.float().cpu(), ro, atol=2e-2, rtol=2e-2)
     torch.testing.assert_close(lse.cpu(), rl, atol=1e-3, rtol=1e-3)
+
+
+@pytest.mark.parametrize("B,S,H,topk,paged", [(1, 9, 16, 31, False), (3, 3, 48, 1100, True), (2, 130, 64, 33, True),
+                                              (120, 1, 32, 1100, True), (1, 120, 64, 1088, False),
+                                              (1, 300, 48, 2049, False)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_up_to_64_heads_tile_and_stage_edges(dsa, dev, B, S, H, topk, paged, dtype):
+    """The 64-head kernel: both ring depths, splits, ragged last tiles, empty tiles, heads short of 64.
+
+    Slots are emptied by -1 and, in a paged cache, by a block of a negative number; key 0 is NaN and
+    never selected, so an empty slot that reads a key instead of zeros shows.
+    """
+    g = torch.Generator().manual_seed(B * S + H + topk)
+    skv, bs = 2112, 64
+    q = (torch.randn(B, S, H, 576, generator=g) * 0.5).to(dtype)
+    kv = (torch.randn(1, skv, 1, 576, generator=g) * 0.5).to(dtype).expand(B, -1, -1, -1).contiguous()
+    idx = torch.stack([1 + torch.randperm(skv - 1, generator=g)[:topk] for _ in range(B * S)])
+    idx = idx.view(B, S, 1, topk).to(torch.int32)
+    idx[:, ::2, :, 3::5] = -1
+    idx[:, 1::3, :, :min(40, topk - 1)] = -1  # the first tile empty
+    idx[:, 2::4, :, topk // 2:] = -1
+    idx[0, S - 1] = -1 if S > 3 else idx[0, S - 1]
+    want_idx, kw = idx, {}
+    kv[:, 0] = float("nan")
+    if paged:
+        # One pool; each sequence its own order of the blocks, block 5 of every sequence missing.
+        pool = kv[0].view(skv // bs, bs, 1, 576)
+        table = torch.arange(skv // bs, dtype=torch.int32).expand(B, -1).contiguous()
+        table[:, 5] = -3
+        want_idx = torch.where((idx >= 0) & (idx // bs == 5), torch.full_like(idx, -1), idx)
+        kw = dict(block_table=table.to(dev))
+    out, lse = dsa.sparse_mla_fwd(q.to(dev), (pool if paged else kv).to(dev), idx.to(dev), 1 / math.sqrt(576), **kw)
+    kv[:, 0] = 0
+    _check(out, lse, *ref.sparse_mla_fwd(q, kv, want_idx, 1 / math.sqrt(576)))

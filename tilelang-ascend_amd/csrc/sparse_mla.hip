@@ -232,6 +232,13 @@ struct TileDma {
       src[ag] = base + (int64_t)row * MlaGeom<kD>::kRowBytes + 16 * ((lane & 7) ^ lds_swizzle(u, a));
     }
   }
+  // One row group per wave, the lane's source address given.
+  __device__ __forceinline__ void prepare_src(const uint8_t* lane_src, uint8_t* stage_base, int wave_) {
+    static_assert(kGroups == 1, "one row group per wave");
+    wave = wave_;
+    stage = stage_base;
+    src[0] = lane_src;
+  }
   template <int D>
   __device__ __forceinline__ void issue() {
     static_assert(D >= 0 && D < kCount, "DMA instruction index");
@@ -1167,17 +1174,17 @@ __device__ __forceinline__ void r4_k_first(u32x4 (&k)[kR4Ahead + 1], const uint3
 }
 // Half-step J of S^T = K Q^T: key half J % 2 of dim step J / 2, accumulator sets
 // by the parity of the step (the sums of qk_half).
-template <bool kF16, bool kDma, int J>
-__device__ __forceinline__ void r4_qk(f32x4 (&c)[2][2], const u32x4 (&qb)[16], const uint32_t (&qa)[2],
-                                      u32x4 (&k)[kR4Ahead + 1], TileDma<kR4Waves, 512>& dma) {
-  constexpr int kHalf = MlaGeom<512>::kQkHalf;
+template <bool kF16, int kD, int kSets, bool kDma, int J>
+__device__ __forceinline__ void r4_qk(f32x4 (&c)[kSets][2], const u32x4 (&qb)[kD / 32], const uint32_t (&qa)[2],
+                                      u32x4 (&k)[kR4Ahead + 1], TileDma<kR4Waves, kD>& dma) {
+  constexpr int kHalf = MlaGeom<kD>::kQkHalf;
   if constexpr (J + kR4Ahead < kHalf) r4_k_read<J + kR4Ahead>(k, qa);
-  if constexpr (kDma) il_dma<kR4Waves, 512, J>(dma);
+  if constexpr (kDma) il_dma<kR4Waves, kD, J>(dma);
   constexpr int kWait = (kHalf - 1 - J) < kR4Ahead ? (kHalf - 1 - J) : kR4Ahead;
   u32x4& kj = k[J % (kR4Ahead + 1)];
   lgkm_wait_k<kWait>(kj);
-  mfma_qk<kF16, (J < 4)>(c[(J / 2) % 2][J % 2], kj, qb[J / 2]);
-  if constexpr (J + 1 < kHalf) r4_qk<kF16, kDma, J + 1>(c, qb, qa, k, dma);
+  mfma_qk<kF16, (J < 2 * kSets)>(c[(J / 2) % kSets][J % 2], kj, qb[J / 2]);
+  if constexpr (J + 1 < kHalf) r4_qk<kF16, kD, kSets, kDma, J + 1>(c, qb, qa, k, dma);
 }
 
 // V group kG (two 16-column blocks) times head block kB of the wave's order (0: its own).
@@ -1316,8 +1323,8 @@ void sparse_mla_rows4_kernel(MlaArgs a) {
     f32x4 c[2][2];
     u32x4 k[kR4Ahead + 1];
     r4_k_first(k, qa);
-    if (more) r4_qk<kF16, true, 0>(c, qb, qa, k, dma);
-    else r4_qk<kF16, false, 0>(c, qb, qa, k, dma);
+    if (more) r4_qk<kF16, 512, 2, true, 0>(c, qb, qa, k, dma);
+    else r4_qk<kF16, 512, 2, false, 0>(c, qb, qa, k, dma);
     static_assert(kR4Ahead + 1 == 3, "the wait below names every K operand register");
     // 24 wait states between the asm MFMAs and the first VALU read of a score (qk_phase).
     __asm__ __volatile__("s_nop 7\n\ts_nop 7\n\ts_nop 7"
@@ -1439,6 +1446,312 @@ void sparse_mla_rows4_kernel(MlaArgs a) {
         *reinterpret_cast<u32x4*>(obase + orow + 32 * p2) =
             u32x4{pack2<kF16>(x[0], x[1]), pack2<kF16>(x[2], x[3]), pack2<kF16>(y[0], y[1]), pack2<kF16>(y[2], y[3])};
       }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The 576-wide index rows at up to 64 heads, in the manner of
+// sparse_mla_rows4_kernel: four waves of 16 heads, O split by output columns,
+// a two-stage ring, two workgroups per CU.  sparse_mla_body at one or two waves
+// (32 heads each) leaves one or two waves on a CU, too few to cover the gather's
+// latency and the softmax; here one workgroup's matrix work covers the other's
+// waits, and the gather itself (9 TB/s out of the caches) is the bound.
+// Two 36 KB stages and P leave no room for a slot table, so each lane looks up
+// the row it will load next as the loop goes, by ordinary loads that the tile's
+// own wait covers.  A scan of the index row beforehand keeps only the tiles'
+// valid-slot masks.  Empty slots load a row of zeros (probability 0 times a stale
+// row's NaN would not be 0).  Measured, 2048 slots a row, us before -> after:
+// 4000 rows of 8000 keys at 16 / 48 / 64 heads 1776 -> 1070, 1690 -> 1075,
+// 1705 -> 1090; 64 decode rows at 16 / 64 heads 51 -> 41, 53 -> 48; 400 rows at
+// 64 heads 236 -> 192.
+// kStages: 3 where a grid has one workgroup per CU anyway and long rows (two tiles
+// in flight; 128 rows at 64 heads 84 -> 76 us, at 16 heads 75 -> 65), else 2.
+template <int kStages>
+struct H64Lds {
+  static constexpr int kMaskOffset = kStages * MlaGeom<576>::kStageBytes + kR4PBytes;
+  static constexpr int kFlagOffset = kMaskOffset + (kSlotsCap / 32) * 4;  // overflow, first and last valid slot
+  static constexpr int kBytes = kFlagOffset + 16;
+};
+static_assert(2 * H64Lds<2>::kBytes <= 160 * 1024, "two workgroups per CU");
+static __device__ __align__(128) uint8_t kMlaZeroRow[MlaGeom<576>::kRowBytes];
+
+template <bool kF16, bool kPaged, int kStages>
+__global__ __launch_bounds__(kR4Waves * kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void sparse_mla_heads64_kernel(MlaArgs a) {
+  constexpr int kD = 576, kSteps = kD / 32;
+  constexpr int kStageBytes = MlaGeom<kD>::kStageBytes;
+  constexpr int kDepth = kStages - 1;  // tiles in flight
+  constexpr int kTileLoads = MlaGeom<kD>::kRowBytes / 128;  // DMA instructions of a wave and tile
+  constexpr int kThreads = kR4Waves * kWave;
+  extern __shared__ __align__(128) uint8_t lds[];
+  uint32_t* tile_mask = reinterpret_cast<uint32_t*>(lds + H64Lds<kStages>::kMaskOffset);
+  int32_t* flags = reinterpret_cast<int32_t*>(lds + H64Lds<kStages>::kFlagOffset);
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int r = lane & 15;
+  const int g = lane >> 4;
+  const int T = a.B * a.S * a.G;
+  const int token = blockIdx.x % T;
+  const int split = blockIdx.x / T;
+  const int bs_row = token / a.G;
+  const int kvg = token - bs_row * a.G;
+  const int b = bs_row / a.S;
+  const int sq = bs_row % a.S;
+  const int head0 = 16 * wave;  // past H the heads repeat H - 1, unstored
+
+  // Every load from a clamped valid address (sparse_mla_body).
+  const int32_t* irow = a.indices + (int64_t)token * a.topk;
+  const int slot_begin = split * a.keys_per_split;
+  const int slot_end = min(a.topk, slot_begin + a.keys_per_split);
+  const int nslots = max(slot_end - slot_begin, 0);
+  const int last_slot = max(slot_end - 1, 0);
+  constexpr int kIdxPerLane = kSlotsCap / kThreads;
+  int idx_raw[kIdxPerLane];
+#pragma unroll
+  for (int j = 0; j < kIdxPerLane; ++j) idx_raw[j] = irow[min(slot_begin + tid + j * kThreads, last_slot)];
+  typedef const __attribute__((address_space(4))) int32_t const_i32;
+  const int ql_raw = a.q_len ? *(const_i32*)(a.q_len + b) : a.S;
+  const int kl_raw = a.kv_len ? *(const_i32*)(a.kv_len + b) : a.Skv;
+  const int ql = min(max(ql_raw, 0), a.S);
+  const int kl = min(max(kl_raw, 0), a.Skv);
+  // Valid: 0 <= idx < kl and idx <= lim; a padded query row has no valid slot.
+  const int bound = sq < ql ? (a.causal ? min(kl - 1, kl - ql + sq) : kl - 1) : -1;
+  const int ntiles_all = (nslots + kMlaTile - 1) / kMlaTile;
+  if (tid == 0) {
+    flags[0] = 0;
+    flags[1] = 0x7fffffff;
+    flags[2] = -1;
+  }
+  // Of a paged cache, slots in blocks of a negative number are empty too.
+  int blk_raw[kIdxPerLane];
+  if constexpr (kPaged) {
+    const int32_t* bt = a.block_table + (int64_t)b * a.max_blocks;
+#pragma unroll
+    for (int j = 0; j < kIdxPerLane; ++j) {
+      const int i = idx_raw[j] >= 0 && idx_raw[j] <= bound ? idx_raw[j] : 0;
+      blk_raw[j] = bt[i / a.block_size];
+    }
+  }
+  __syncthreads();
+  int wave_first = 0x7fffffff, wave_last = -1;
+#pragma unroll
+  for (int j = 0; j < kIdxPerLane; ++j) {
+    const int i0 = wave * kWave + j * kThreads;
+    const bool ok = i0 + lane < nslots && idx_raw[j] >= 0 && idx_raw[j] <= bound;
+    const uint64_t vm = __ballot(ok && (!kPaged || blk_raw[j] >= 0));
+    if (vm != 0) {
+      wave_first = min(wave_first, i0 + (int)__builtin_ctzll(vm));
+      wave_last = max(wave_last, i0 + 63 - (int)__builtin_clzll(vm));
+    }
+    if (lane == 0 && i0 < ntiles_all * kMlaTile) {
+      tile_mask[i0 / kMlaTile] = (uint32_t)vm;
+      if (i0 / kMlaTile + 1 < ntiles_all) tile_mask[i0 / kMlaTile + 1] = (uint32_t)(vm >> 32);
+    }
+  }
+  if (lane == 0 && wave_first != 0x7fffffff) {
+    atomicMin(&flags[1], wave_first);
+    atomicMax(&flags[2], wave_last);
+  }
+  __syncthreads();
+  const int fv = flags[1], lv = flags[2];
+  const int t_first = lv < 0 ? 0 : fv / kMlaTile;
+  const int ntiles = lv < 0 ? 0 : lv / kMlaTile + 1 - t_first;  // no valid slot: out = 0, lse = -inf
+  const uint32_t* tmask = tile_mask + t_first;
+
+  // This lane's slot of tile t (of the t_first ..): 32 t + 8 wave + lane / 8.
+  const int lane_slot = t_first * kMlaTile + 8 * wave + (lane >> 3);
+  auto load_idx = [&](int t) { return irow[min(slot_begin + lane_slot + t * kMlaTile, last_slot)]; };
+  auto slot_valid = [&](int t, int idx, int blk) {
+    return lane_slot + t * kMlaTile < nslots && idx >= 0 && idx <= bound && blk >= 0;
+  };
+  auto load_blk = [&](int idx) {
+    if constexpr (kPaged) {
+      const int i = idx >= 0 && idx <= bound ? idx : 0;
+      return a.block_table[(int64_t)b * a.max_blocks + i / a.block_size];
+    } else {
+      return 0;
+    }
+  };
+  const uint32_t chunk = 16 * ((lane & 7) ^ lds_swizzle(lane >> 3, wave));
+  const uint8_t* zero_row = kMlaZeroRow;
+  __asm__("" : "+s"(zero_row));  // the address is kept, not looked up again for each tile
+  auto lane_src = [&](int t, int idx, int blk) -> const uint8_t* {
+    const int64_t row = kPaged ? ((int64_t)blk * a.block_size + idx % a.block_size) * a.G + kvg
+                               : ((int64_t)b * a.Skv + idx) * a.G + kvg;
+    const uint8_t* p = reinterpret_cast<const uint8_t*>(a.kv) + row * MlaGeom<kD>::kRowBytes;
+    return (slot_valid(t, idx, blk) ? p : zero_row) + chunk;
+  };
+  // The rows of tile t + kDepth go out in iteration t, looked up in the one before.
+  int idx_n = 0, idx_nn = 0, blk_n = 0;
+  u32x4 qb[kSteps];
+  {
+    const uint16_t* qp = a.q + ((int64_t)token * a.H + min(head0 + r, a.H - 1)) * kD + 8 * g;
+    int idx[kStages], blk[kStages];
+    if (ntiles > 0) {
+#pragma unroll
+      for (int t = 0; t < kStages; ++t) idx[t] = load_idx(t);
+      idx_nn = load_idx(kStages);
+#pragma unroll
+      for (int t = 0; t < kStages; ++t) blk[t] = load_blk(idx[t]);
+      TileDma<kR4Waves, kD> dma;
+      dma.prepare_src(lane_src(0, idx[0], blk[0]), lds, wave);
+      il_dma_all(dma);
+    }
+    // Q before the last tile in flight: the loop's first wait covers it.
+#pragma unroll
+    for (int st = 0; st < kSteps; ++st) qb[st] = *reinterpret_cast<const u32x4*>(qp + 32 * st);
+    if (ntiles > 0) {
+      if constexpr (kDepth == 2) {
+        __asm__ __volatile__("" ::: "memory");
+        TileDma<kR4Waves, kD> dma;
+        dma.prepare_src(lane_src(1, idx[1], blk[1]), lds + kStageBytes, wave);
+        il_dma_all(dma);
+      }
+      idx_n = idx[kDepth];
+      blk_n = blk[kDepth];
+    }
+  }
+
+  f32x4 o[4][8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_ref = -__builtin_huge_valf(), lsum = 0.f;
+  bool overflow = false;
+  const float scale_log2 = a.scale_log2;
+  const uint32_t qk_lane = 1024 * (r >> 3) + 128 * (r & 7) + 16 * (g ^ lds_swizzle(r & 7, r >> 3));
+  const int pv_u = 4 * (g & 1) + (r >> 2);
+  const uint32_t pv_lane = 1024 * (g >> 1) + 128 * pv_u + 16 * ((r & 3) ^ lds_swizzle(pv_u, g >> 1)) + 8192 * wave;
+  const uint32_t p_base = lds_u32(lds + kStages * kStageBytes) + 16 * lane;
+
+  int stage = 0, fill = kDepth * kStageBytes;  // of tile and tile + kDepth
+  for (int tile = 0; tile < ntiles; ++tile) {
+    // Tile, Q, and the last iteration's lookups (issued before its DMA) have arrived;
+    // the barrier publishes the tile and certifies that every wave is done with the
+    // last one and its P.
+    wait_vmcnt<(kDepth - 1) * kTileLoads>();
+    raw_barrier();
+    // Past the last tile every slot is empty: the zero row, into a stage no one reads.
+    TileDma<kR4Waves, kD> dma;
+    dma.prepare_src(lane_src(tile + kDepth, idx_n, blk_n), lds + fill, wave);
+    blk_n = load_blk(idx_nn);
+    // A move of its own: one the compiler places may come after the load below and wait for it.
+    __asm__ __volatile__("v_mov_b32 %0, %1" : "=v"(idx_n) : "v"(idx_nn));
+    idx_nn = load_idx(tile + kDepth + 2);
+    const uint32_t mask = __builtin_amdgcn_readfirstlane(tmask[tile]);
+    const uint32_t base = lds_u32(lds) + stage;
+    stage = stage == kDepth * kStageBytes ? 0 : stage + kStageBytes;
+    fill = fill == kDepth * kStageBytes ? 0 : fill + kStageBytes;
+    if constexpr (kDepth == 2) __builtin_amdgcn_sched_barrier(0);  // the lookups before the DMA
+    const uint32_t qa[2] = {base + qk_lane, (base + qk_lane) ^ 64};
+    f32x4 c[1][2];
+    u32x4 k[kR4Ahead + 1];
+    r4_k_first(k, qa);
+    r4_qk<kF16, kD, 1, true, 0>(c, qb, qa, k, dma);
+    static_assert(kR4Ahead + 1 == 3, "the wait below names every K operand register");
+    // 24 wait states between the asm MFMAs and the first VALU read of a score (qk_phase).
+    __asm__ __volatile__("s_nop 7\n\ts_nop 7\n\ts_nop 7"
+                         : "+v"(c[0][0]), "+v"(c[0][1]), "+v"(k[0]), "+v"(k[1]), "+v"(k[2]));
+    float s[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s[e] = c[0][e / 4][e % 4];
+    if (mask != 0xffffffffu) {
+      const uint32_t bits = ((mask >> (4 * g)) & 15u) | (((mask >> (16 + 4 * g)) & 15u) << 4);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s[e] = ((bits >> e) & 1u) ? s[e] : -__builtin_huge_valf();
+    }
+    if (tile == 0) {  // holds the first valid slot: fixes the reference
+      float cmax = s[0];
+#pragma unroll
+      for (int e = 1; e < 8; ++e) cmax = fmaxf(cmax, s[e]);
+      cmax = fmaxf(cmax, __shfl_xor(cmax, 16, kWave));
+      cmax = fmaxf(cmax, __shfl_xor(cmax, 32, kWave));
+      m_ref = cmax * scale_log2 + PRange<kF16>::kRefBias;
+    }
+    const float neg_m = -m_ref;
+    float p[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) p[e] = fast_exp2(fmaf(s[e], scale_log2, neg_m));
+    const float ps = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+    lsum += ps;
+    overflow = overflow || !(ps <= kOverflowSumOf<kF16>);
+    const u32x4 pa = {pack2<kF16>(p[0], p[1]), pack2<kF16>(p[2], p[3]), pack2<kF16>(p[4], p[5]),
+                      pack2<kF16>(p[6], p[7])};
+    r4_p_write(pa, p_base + 1024 * wave);
+    const uint32_t va[2] = {base + pv_lane, (base + pv_lane) ^ 64};
+    u32x2 v[2][4];
+    pv_group_reads<0>(v[0], va);
+    lgkm_wait<0>(v[0]);  // P is written too
+    raw_barrier();
+    u32x4 px[3];
+    b128_read<0>(px[0], p_base + 1024 * ((wave + 1) & 3));
+    b128_read<0>(px[1], p_base + 1024 * ((wave + 2) & 3));
+    b128_read<0>(px[2], p_base + 1024 * ((wave + 3) & 3));
+    pv_group_reads<1>(v[1], va);
+    r4_pv<kF16, 0, 0>(o, v[0], pa);
+    lgkm_wait_k<6>(px[0]);
+    r4_pv<kF16, 0, 1>(o, v[0], px[0]);
+    lgkm_wait_k<5>(px[1]);
+    r4_pv<kF16, 0, 2>(o, v[0], px[1]);
+    lgkm_wait_k<4>(px[2]);
+    r4_pv<kF16, 0, 3>(o, v[0], px[2]);
+    r4_pv_group<kF16, 1>(o, v, va, pa, px);
+    r4_pv_group<kF16, 2>(o, v, va, pa, px);
+    r4_pv_group<kF16, 3>(o, v, va, pa, px);
+  }
+  // All LDS reads and loads retire before the ring is reused below.
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (__any(overflow) && lane == 0) flags[0] = 1;
+  __syncthreads();
+  const bool final_out = a.splits == 1;
+  uint16_t* obase = final_out ? a.out : a.part_o + (int64_t)split * T * a.H * kMlaDV;
+  float* lbase = final_out ? a.lse : a.part_lse + (int64_t)split * T * a.H;
+  if (flags[0]) {
+    // Scores that outgrew the reference: the exact path, over a slot table made now.
+    int32_t* rows = reinterpret_cast<int32_t*>(lds + 2 * kSlotsCap * 4);
+    for (int i = tid; i < ntiles_all * kMlaTile; i += kThreads) {
+      const int idx = irow[min(slot_begin + i, last_slot)];
+      const bool ok = i < nslots && idx >= 0 && idx <= bound;
+      const int at = ok ? idx : 0;  // a negative block number makes the row negative: empty
+      const int row = kPaged ? (a.block_table[(int64_t)b * a.max_blocks + at / a.block_size] * a.block_size +
+                                at % a.block_size) * a.G + kvg
+                             : (b * a.Skv + at) * a.G + kvg;
+      rows[i] = ok ? row : -1;
+    }
+    __syncthreads();
+    mla_exact_fallback<kF16, kD>(a.q, reinterpret_cast<const uint8_t*>(a.kv), nullptr, nullptr, obase, nullptr, lbase,
+                                 a.H, scale_log2, rows, ntiles_all * kMlaTile, token, 0, kR4Heads,
+                                 reinterpret_cast<float*>(lds), kThreads);
+    return;
+  }
+  {
+    float l_tot = lsum;
+    l_tot += __shfl_xor(l_tot, 16, kWave);
+    l_tot += __shfl_xor(l_tot, 32, kWave);
+    if (g == 0) {
+      reinterpret_cast<float*>(lds)[16 * wave + r] = l_tot > 0.f ? 1.f / l_tot : 0.f;
+      if (head0 + r < a.H)
+        lbase[(int64_t)token * a.H + head0 + r] =
+            l_tot > 0.f ? (m_ref + fast_log2(l_tot)) * 0.69314718055994531f : -__builtin_huge_valf();
+    }
+  }
+  __syncthreads();
+  const int col0 = 128 * wave + 8 * g;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int hb = 16 * ((wave + i) & 3);
+    const float inv = reinterpret_cast<const float*>(lds)[hb + r];
+    if (hb >= a.H) continue;  // wave-uniform
+    const int64_t orow = ((int64_t)token * a.H + hb + r) * kMlaDV + col0;
+#pragma unroll
+    for (int p2 = 0; p2 < 4; ++p2) {
+      const f32x4 x = o[i][2 * p2] * inv, y = o[i][2 * p2 + 1] * inv;
+      *reinterpret_cast<u32x4*>(obase + orow + 32 * p2) =
+          u32x4{pack2<kF16>(x[0], x[1]), pack2<kF16>(x[2], x[3]), pack2<kF16>(y[0], y[1]), pack2<kF16>(y[2], y[3])};
     }
   }
 }
@@ -1660,6 +1973,27 @@ static hipError_t launch_mla_kernel(const MlaArgs& a, int head_groups, hipStream
   return hipGetLastError();
 }
 
+template <bool kF16>
+static hipError_t launch_mla_heads64(const MlaArgs& a, hipStream_t stream) {
+  const int64_t wgs = (int64_t)a.B * a.S * a.G * a.splits;
+  const auto launch = [&](auto paged, auto stages) {
+    constexpr bool kPaged = decltype(paged)::value;
+    constexpr int kStages = decltype(stages)::value;
+    constexpr int kLds = H64Lds<kStages>::kBytes;
+    const hipError_t e = set_dynamic_lds_once<sparse_mla_heads64_kernel<kF16, kPaged, kStages>>(kLds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((sparse_mla_heads64_kernel<kF16, kPaged, kStages>), dim3((unsigned)wgs), dim3(kR4Waves * kWave),
+                       kLds, stream, a);
+    return hipGetLastError();
+  };
+  const auto paged = [&](auto stages) {
+    return a.block_table ? launch(std::true_type{}, stages) : launch(std::false_type{}, stages);
+  };
+  // One workgroup per CU at most: the third stage is free, and pays past 16 tiles a
+  // workgroup (at 4 or 16 tiles both take the same time, within 1 us).
+  return wgs <= 256 && a.keys_per_split > 16 * kMlaTile ? paged(std::integral_constant<int, 3>{}) : paged(std::integral_constant<int, 2>{});
+}
+
 // Row lists (D = 512) never use a block table.
 template <int kNW, bool kF16, int kD>
 static hipError_t launch_mla_nw(const MlaArgs& a, int head_groups, hipStream_t stream) {
@@ -1672,9 +2006,13 @@ static hipError_t launch_mla_nw(const MlaArgs& a, int head_groups, hipStream_t s
 template <bool kF16, int kD>
 static hipError_t launch_mla_dtype(const MlaArgs& a, int head_groups, int hpg, hipStream_t stream) {
   hipError_t e;
-  if (hpg > 64) e = launch_mla_nw<4, kF16, kD>(a, head_groups, stream);
-  else if (hpg > 32) e = launch_mla_nw<2, kF16, kD>(a, head_groups, stream);
-  else e = launch_mla_nw<1, kF16, kD>(a, head_groups, stream);
+  if constexpr (kD == 576) {
+    e = hpg <= kR4Heads ? launch_mla_heads64<kF16>(a, stream) : launch_mla_nw<4, kF16, kD>(a, head_groups, stream);
+  } else {
+    if (hpg > 64) e = launch_mla_nw<4, kF16, kD>(a, head_groups, stream);
+    else if (hpg > 32) e = launch_mla_nw<2, kF16, kD>(a, head_groups, stream);
+    else e = launch_mla_nw<1, kF16, kD>(a, head_groups, stream);
+  }
   if (e != hipSuccess || a.splits == 1) return e;
   const int64_t rows = (int64_t)a.B * a.S * a.G * a.H;
   const int64_t threads = rows * (kMlaDV / 8);
