@@ -277,11 +277,11 @@ def test_decode_parts_equal_the_joined_call(dsa, dev, T, N, topk, nb, dtype):
         assert torch.equal(out, same)
 
 
-@pytest.mark.parametrize("h", [32, 48, 64, 80])
+@pytest.mark.parametrize("h", [16, 32, 48, 64, 80])
 @pytest.mark.parametrize("topk", [1, 31, 33, 200, 2080])
 def test_row_lists_head_and_tile_edges(dsa, dev, h, topk):
-    """More than 8 rows, so the row-list kernels: both sides of their head counts (one wave, four waves
-    of 16 heads with a missing and with every block, four of 32) by list lengths of less than a tile, a
+    """More than 8 rows, so the row-list kernels: both sides of their head counts (four waves of 16
+    heads with missing blocks and with every block, four of 32) by list lengths of less than a tile, a
     tile and one row, many tiles, and more slots than one workgroup holds (split partials); -1 slots
     leave the first, a middle or every tile of some rows empty.  Bars as the module's bf16 ones."""
     g = torch.Generator().manual_seed(h + topk)

@@ -12,8 +12,8 @@
 // (example_sparse_flash_attn_mask_pa.py:226-233).  LSE convention:
 // examples/deepseek_v4/sparse_flash_mla/sparse_flash_mla_golden.py:149.
 //
-// Work split.  One workgroup per (query row, split of the index list, group
-// of up to 128 heads); a wave owns 32 heads (two 16-head MFMA blocks that share
+// Work split, more than 64 heads.  One workgroup of four waves per (query row, split
+// of the index list, group of up to 128 heads); a wave owns 32 heads (two 16-head MFMA blocks that share
 // every K and V operand read from LDS) and keeps their Q rows in registers, the
 // O accumulators (32 x 512 fp32) in AGPRs: one wave per SIMD.
 //
@@ -43,10 +43,8 @@
 // into slices between them.  With more than one split a workgroup writes a
 // normalised bf16 partial and its LSE; a combine kernel merges them.
 //
-// The 512-wide row lists of up to 32 heads (one wave) run the same body from a
-// two-stage ring instead (sparse_mla_rows2_kernel): one tile is computed at a
-// time while the next arrives, in 73 KB of LDS, so that two workgroups share a
-// CU.  Those of 33 to 64 heads have a kernel of their own (sparse_mla_rows4_kernel).
+// Up to 64 heads have kernels of their own, two workgroups to a CU: the 512-wide row
+// lists sparse_mla_rows4_kernel, the 576-wide index rows sparse_mla_heads64_kernel.
 #include "common.hpp"
 
 namespace dsa {
@@ -623,18 +621,11 @@ __device__ __attribute__((noinline)) void mla_exact_fallback(const uint16_t* q, 
 }
 
 // kPaged: the KV rows are addressed through a block table (a.block_table).
-// kSt: ring stages.  4 (sparse_mla_kernel): the pipelined loop below.  2
-// (sparse_mla_rows2_kernel: the 512-wide row lists with one wave, i.e. up to 32
-// heads): each tile is computed in turn -- Q K^T, softmax, P V -- while the
-// next tile's DMA fills the other stage; the 73 KB of LDS let two workgroups
-// share a CU, and each workgroup's exposed DMA latency, prologue and epilogue
-// overlap the other's.
-template <int kNW, bool kF16, int kD, bool kPaged, int kSt>
-__device__ __forceinline__ void sparse_mla_body(MlaArgs a) {
-  static_assert(kSt == kStages || kSt == 2, "ring stages");
+template <int kNW, bool kF16, int kD, bool kPaged>
+__global__ __launch_bounds__(kNW * kWave) void sparse_mla_kernel(MlaArgs a) {
   using Cfg = MlaCfg<kNW, kD>;
   using Geo = MlaGeom<kD>;
-  using Lay = MlaLayout<kD, kSt>;
+  using Lay = MlaLayout<kD, kStages>;
   extern __shared__ __align__(16) uint8_t lds[];
   int32_t* rows = reinterpret_cast<int32_t*>(lds + Lay::kRowsOffset);
   const int tid = threadIdx.x;
@@ -824,12 +815,12 @@ __device__ __forceinline__ void sparse_mla_body(MlaArgs a) {
       pv_lane[par] = 1024 * (g >> 1) + 128 * u + 16 * ((4 * par + (r & 3)) ^ lds_swizzle(u, g >> 1));
   }
   auto stage_k = [&](int tile, uint32_t (&out)[2]) {
-    const uint32_t base = lds_u32(lds + (tile % kSt) * kStageBytes);
+    const uint32_t base = lds_u32(lds + (tile % kStages) * kStageBytes);
     out[0] = base + qk_lane[0];
     out[1] = base + qk_lane[1];
   };
   auto stage_v = [&](int tile, uint32_t (&out)[2]) {
-    const uint32_t base = lds_u32(lds + (tile % kSt) * kStageBytes);
+    const uint32_t base = lds_u32(lds + (tile % kStages) * kStageBytes);
     out[0] = base + pv_lane[0];
     out[1] = base + pv_lane[1];
   };
@@ -867,58 +858,7 @@ __device__ __forceinline__ void sparse_mla_body(MlaArgs a) {
   // softmax turns S(t+1) into P(t+1) (phase B).  One barrier per tile: it
   // publishes tile t+1 and certifies that every wave is done with tile t-1,
   // whose stage the DMA of tile t + kDepth then refills.
-  if (kSt == 2 && ntiles > 0) {
-    // Two stages: tile t in stage t & 1; the DMA of tile t + 1 goes out spread
-    // over the Q K^T of tile t, into the stage tile t - 1 left.
-    {
-      TileDma<kNW, kD> dma;
-      dma.prepare(kvb, kvb2, trows, safe_row, 0, lds, wave, lane);
-      il_dma_all(dma);
-    }
-    u32x4 pa[2];
-    for (int tile = 0; tile < ntiles; ++tile) {
-      // Tile `tile` has arrived (vector-memory loads complete in order, so this
-      // also covers Q); the barrier publishes it and certifies that every wave
-      // is done with tile - 1.
-      wait_vmcnt<0>();
-      raw_barrier();
-      const bool more = tile + 1 < ntiles;  // workgroup-uniform
-      TileDma<kNW, kD> dma;
-      if (more) dma.prepare(kvb, kvb2, trows, safe_row, tile + 1, lds + ((tile + 1) % kSt) * kStageBytes, wave, lane);
-      f32x4 c[2][2];
-      uint32_t qa[2], va[2];
-      stage_k(tile, qa);
-      stage_v(tile, va);
-      if (more) qk_phase<kF16, kNW, kD, true>(c, qb, qa, dma);
-      else qk_phase<kF16, kNW, kD, false>(c, qb, qa, dma);
-      mask_scores(c, __builtin_amdgcn_readfirstlane(tmask[tile]));
-      if (tile == 0) {
-        // The first processed tile holds the first valid slot: it fixes m_ref.
-#pragma unroll
-        for (int hb = 0; hb < 2; ++hb) {
-          float cmax = -__builtin_huge_valf();
-#pragma unroll
-          for (int e = 0; e < 8; ++e) cmax = fmaxf(cmax, c[hb][e / 4][e % 4]);
-          cmax = fmaxf(cmax, __shfl_xor(cmax, 16, kWave));
-          cmax = fmaxf(cmax, __shfl_xor(cmax, 32, kWave));
-          m_ref[hb] = cmax * scale_log2 + PRange<kF16>::kRefBias;
-        }
-      }
-      Softmax sm{c, pa, lsum, lsum_r, overflow, {-m_ref[0], -m_ref[1]}, scale_log2, {}};
-      sm.template run<0>();
-      sm.template run<1>();
-      sm.template run<2>();
-      sm.template run<3>();
-      sm.template run<4>();
-      sm.template run<5>();
-      sm.template run<6>();
-      sm.template run<7>();
-      sm.template run<8>();
-      sm.template run<9>();
-      pv_only<kF16>(o, pa, va);
-    }
-  }
-  if (kSt == kStages && ntiles > 0) {
+  if (ntiles > 0) {
     // The first kDepth stages are filled now (a row of fewer tiles re-loads its
     // last tile into the stages it does not use), unconditionally, so that the
     // compiler sees a fixed count of loads behind Q: the wait for tile 0 then
@@ -1125,18 +1065,8 @@ __device__ __forceinline__ void sparse_mla_body(MlaArgs a) {
           ltot_h[hb] > 0.f ? (mout_h[hb] + fast_log2(ltot_h[hb])) * 0.69314718055994531f : -__builtin_huge_valf();
 }
 
-template <int kNW, bool kF16, int kD, bool kPaged>
-__global__ __launch_bounds__(kNW * kWave) void sparse_mla_kernel(MlaArgs a) {
-  sparse_mla_body<kNW, kF16, kD, kPaged, kStages>(a);
-}
-
-template <bool kF16>
-__global__ __launch_bounds__(kWave) void sparse_mla_rows2_kernel(MlaArgs a) {
-  sparse_mla_body<1, kF16, 512, false, 2>(a);
-}
-
 // ---------------------------------------------------------------------------
-// The 512-wide row lists of 33 to 64 heads: four waves of 16 heads, two waves
+// The 512-wide row lists of up to 64 heads: four waves of 16 heads, two waves
 // per SIMD.  A tile is computed in turn -- Q K^T, softmax, P V -- from a
 // two-stage ring while the next tile's DMA fills the other stage, and nothing
 // inside a wave overlaps these; a second wave on its SIMD (the workgroup has a
@@ -1147,6 +1077,10 @@ __global__ __launch_bounds__(kWave) void sparse_mla_rows2_kernel(MlaArgs a) {
 // x 32 keys a wave) through LDS.  Against one wave per SIMD of 32 heads each, 8192
 // rows by 64 heads, row lists included: window + 512 selected rows 783 -> 666 us,
 // window alone 359 -> 294, window + 64 dense rows 414 -> 347 (outputs bit-equal).
+// At 16 and 32 heads some waves repeat others' work, yet against one wave of 32
+// heads a workgroup (two workgroups per CU): window + 512 selected, 4096 rows,
+// 423 -> 355 and 429 -> 368 us; window alone, 8192 rows, 309 -> 206 and 330 -> 243;
+// 64 decode rows 57 -> 50 and 59 -> 51 (bit-equal too).
 constexpr int kR4Waves = 4;
 constexpr int kR4Heads = 64;                            // heads per workgroup
 constexpr int kR4PBytes = kR4Waves * 1024;              // one P operand per wave
@@ -1224,10 +1158,9 @@ void sparse_mla_rows4_kernel(MlaArgs a) {
   const int T = a.B * a.S;
   const int token = blockIdx.x % T;
   const int split = blockIdx.x / T;
-  const int group0 = blockIdx.y * kR4Heads;
-  const int head0 = group0 + 16 * wave;  // this wave's Q K^T heads; past H they repeat head H - 1, unstored
+  const int head0 = 16 * wave;  // this wave's Q K^T heads; past H they repeat head H - 1, unstored
 
-  // Slots first, then Q (as in sparse_mla_body): every load from a clamped valid address.
+  // Slots first, then Q (as in sparse_mla_kernel): every load from a clamped valid address.
   const int32_t* irow = a.indices + (int64_t)token * a.topk;
   const int slot_begin = split * a.keys_per_split;
   const int count_raw = a.slot_count[token];  // negative: a padded query row (out = 0, lse = 0)
@@ -1278,7 +1211,7 @@ void sparse_mla_rows4_kernel(MlaArgs a) {
   }
   __syncthreads();
   // Leading and trailing tiles without a valid slot are skipped; the first valid
-  // slot's row stands in for empty ones (sparse_mla_body).
+  // slot's row stands in for empty ones (sparse_mla_kernel).
   const int fv = *first_valid;
   const int safe_row = fv < kSlotsCap ? rows[fv] : -1;
   const int nslots_all = ntiles * kMlaTile;
@@ -1297,7 +1230,7 @@ void sparse_mla_rows4_kernel(MlaArgs a) {
   float m_ref = -__builtin_huge_valf(), lsum = 0.f, lsum_r = 0.f;
   bool overflow = false;
   const float scale_log2 = a.scale_log2;
-  // Operand addresses in a stage (sparse_mla_body); odd steps and column pairs differ in bit 6 alone.
+  // Operand addresses in a stage (sparse_mla_kernel); odd steps and column pairs differ in bit 6 alone.
   const uint32_t qk_lane = 1024 * (r >> 3) + 128 * (r & 7) + 16 * (g ^ lds_swizzle(r & 7, r >> 3));
   const int pv_u = 4 * (g & 1) + (r >> 2);
   const uint32_t pv_lane = 1024 * (g >> 1) + 128 * pv_u + 16 * ((r & 3) ^ lds_swizzle(pv_u, g >> 1)) + 8192 * wave;
@@ -1393,10 +1326,10 @@ void sparse_mla_rows4_kernel(MlaArgs a) {
   const float* sinks = final_out ? a.sinks : nullptr;  // else they join in the combine
   if (*overflow_flag) {
     mla_exact_fallback<kF16, 512>(a.q, kvb, kvb2, sinks, obase, obase32, lbase, a.H, scale_log2, rows, nslots_all, token,
-                                  group0, kR4Heads, reinterpret_cast<float*>(lds), kThreads);
+                                  0, kR4Heads, reinterpret_cast<float*>(lds), kThreads);
     return;
   }
-  // Normalisers of this wave's heads (sparse_mla_body's: O by the rounded weights,
+  // Normalisers of this wave's heads (sparse_mla_kernel's: O by the rounded weights,
   // the LSE by the exact sum, the sink in both), then round to every wave.
   {
     float l_tot = lsum, l_r = lsum_r;
@@ -1434,8 +1367,8 @@ void sparse_mla_rows4_kernel(MlaArgs a) {
   for (int b = 0; b < 4; ++b) {
     const int hb = 16 * ((wave + b) & 3);
     const float inv = reinterpret_cast<const float*>(lds)[hb + r];
-    if (group0 + hb >= a.H) continue;  // wave-uniform
-    const int64_t orow = ((int64_t)token * a.H + group0 + hb + r) * kMlaDV + col0;
+    if (hb >= a.H) continue;  // wave-uniform
+    const int64_t orow = ((int64_t)token * a.H + hb + r) * kMlaDV + col0;
 #pragma unroll
     for (int p2 = 0; p2 < 4; ++p2) {
       const f32x4 x = o[b][2 * p2] * inv, y = o[b][2 * p2 + 1] * inv;
@@ -1453,8 +1386,8 @@ void sparse_mla_rows4_kernel(MlaArgs a) {
 // ---------------------------------------------------------------------------
 // The 576-wide index rows at up to 64 heads, in the manner of
 // sparse_mla_rows4_kernel: four waves of 16 heads, O split by output columns,
-// a two-stage ring, two workgroups per CU.  sparse_mla_body at one or two waves
-// (32 heads each) leaves one or two waves on a CU, too few to cover the gather's
+// a two-stage ring, two workgroups per CU.  sparse_mla_kernel at one or two waves
+// (32 heads each) left one or two waves on a CU, too few to cover the gather's
 // latency and the softmax; here one workgroup's matrix work covers the other's
 // waits, and the gather itself (9 TB/s out of the caches) is the bound.
 // Two 36 KB stages and P leave no room for a slot table, so each lane looks up
@@ -1501,7 +1434,7 @@ void sparse_mla_heads64_kernel(MlaArgs a) {
   const int sq = bs_row % a.S;
   const int head0 = 16 * wave;  // past H the heads repeat H - 1, unstored
 
-  // Every load from a clamped valid address (sparse_mla_body).
+  // Every load from a clamped valid address (sparse_mla_kernel).
   const int32_t* irow = a.indices + (int64_t)token * a.topk;
   const int slot_begin = split * a.keys_per_split;
   const int slot_end = min(a.topk, slot_begin + a.keys_per_split);
@@ -1951,25 +1884,22 @@ hipError_t mla_scratch_ptr(void** out) {
   return result[dev];
 }
 
-template <int kNW, bool kF16, int kD, bool kPaged>
+template <bool kF16, int kD, bool kPaged>
 static hipError_t launch_mla_kernel(const MlaArgs& a, int head_groups, hipStream_t stream) {
   const dim3 grid((unsigned)((int64_t)a.B * a.S * a.G * a.splits), (unsigned)head_groups);
-  if constexpr (kD == 512 && kNW == 2) {
-    const hipError_t ea = set_dynamic_lds_once<sparse_mla_rows4_kernel<kF16>>(kR4Lds);
-    if (ea != hipSuccess) return ea;
-    hipLaunchKernelGGL((sparse_mla_rows4_kernel<kF16>), grid, dim3(kR4Waves * kWave), kR4Lds, stream, a);
-  } else if constexpr (kD == 512 && kNW == 1) {
-    // Two-stage ring for the 512-wide row lists of up to 32 heads (see the kernel).
-    constexpr int kLds = MlaLayout<512, 2>::kLds;
-    const hipError_t ea = set_dynamic_lds_once<sparse_mla_rows2_kernel<kF16>>(kLds);
-    if (ea != hipSuccess) return ea;
-    hipLaunchKernelGGL((sparse_mla_rows2_kernel<kF16>), grid, dim3(kWave), kLds, stream, a);
-  } else {
-    constexpr int kLds = MlaLayout<kD, kStages>::kLds;
-    const hipError_t ea = set_dynamic_lds_once<sparse_mla_kernel<kNW, kF16, kD, kPaged>>(kLds);
-    if (ea != hipSuccess) return ea;
-    hipLaunchKernelGGL((sparse_mla_kernel<kNW, kF16, kD, kPaged>), grid, dim3(kNW * kWave), kLds, stream, a);
-  }
+  constexpr int kNW = 4, kLds = MlaLayout<kD, kStages>::kLds;
+  const hipError_t e = set_dynamic_lds_once<sparse_mla_kernel<kNW, kF16, kD, kPaged>>(kLds);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((sparse_mla_kernel<kNW, kF16, kD, kPaged>), grid, dim3(kNW * kWave), kLds, stream, a);
+  return hipGetLastError();
+}
+
+template <bool kF16>
+static hipError_t launch_mla_rows4(const MlaArgs& a, hipStream_t stream) {
+  const dim3 grid((unsigned)((int64_t)a.B * a.S * a.G * a.splits));
+  const hipError_t e = set_dynamic_lds_once<sparse_mla_rows4_kernel<kF16>>(kR4Lds);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((sparse_mla_rows4_kernel<kF16>), grid, dim3(kR4Waves * kWave), kR4Lds, stream, a);
   return hipGetLastError();
 }
 
@@ -1991,27 +1921,22 @@ static hipError_t launch_mla_heads64(const MlaArgs& a, hipStream_t stream) {
   };
   // One workgroup per CU at most: the third stage is free, and pays past 16 tiles a
   // workgroup (at 4 or 16 tiles both take the same time, within 1 us).
-  return wgs <= 256 && a.keys_per_split > 16 * kMlaTile ? paged(std::integral_constant<int, 3>{}) : paged(std::integral_constant<int, 2>{});
+  return wgs <= 256 && a.keys_per_split > 16 * kMlaTile ? paged(std::integral_constant<int, 3>{})
+                                                        : paged(std::integral_constant<int, 2>{});
 }
 
-// Row lists (D = 512) never use a block table.
-template <int kNW, bool kF16, int kD>
-static hipError_t launch_mla_nw(const MlaArgs& a, int head_groups, hipStream_t stream) {
-  if constexpr (kD == 576) {
-    if (a.block_table) return launch_mla_kernel<kNW, kF16, kD, true>(a, head_groups, stream);
-  }
-  return launch_mla_kernel<kNW, kF16, kD, false>(a, head_groups, stream);
-}
-
+// Up to 64 heads (hpg) the 64-head kernels, where their measurements stand; past that
+// they would gather every row twice (576 wide, 128 heads as two groups: 64 decode rows
+// 62 -> 73 us).  Row lists (D = 512) never use a block table.
 template <bool kF16, int kD>
 static hipError_t launch_mla_dtype(const MlaArgs& a, int head_groups, int hpg, hipStream_t stream) {
   hipError_t e;
   if constexpr (kD == 576) {
-    e = hpg <= kR4Heads ? launch_mla_heads64<kF16>(a, stream) : launch_mla_nw<4, kF16, kD>(a, head_groups, stream);
+    if (hpg <= kR4Heads) e = launch_mla_heads64<kF16>(a, stream);
+    else if (a.block_table) e = launch_mla_kernel<kF16, kD, true>(a, head_groups, stream);
+    else e = launch_mla_kernel<kF16, kD, false>(a, head_groups, stream);
   } else {
-    if (hpg > 64) e = launch_mla_nw<4, kF16, kD>(a, head_groups, stream);
-    else if (hpg > 32) e = launch_mla_nw<2, kF16, kD>(a, head_groups, stream);
-    else e = launch_mla_nw<1, kF16, kD>(a, head_groups, stream);
+    e = hpg <= kR4Heads ? launch_mla_rows4<kF16>(a, stream) : launch_mla_kernel<kF16, kD, false>(a, head_groups, stream);
   }
   if (e != hipSuccess || a.splits == 1) return e;
   const int64_t rows = (int64_t)a.B * a.S * a.G * a.H;
