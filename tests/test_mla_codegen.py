@@ -52,3 +52,16 @@ def test_no_spill_in_the_tile_loop(asm):
                 assert "scratch_" not in line, f"{name}: spill in the tile loop: {line}"
         checked += 1
     assert checked >= 4
+
+
+def test_no_spill_in_the_64_head_tile_loops(asm):
+    """The two-workgroup kernels sit at their 256 registers: a reload in the loop would wait for the DMA."""
+    names = re.findall(r"^(_ZN3dsa\d+sparse_mla_(?:rows4|heads64)_kernel\S+):", asm, re.M)
+    assert len(names) == 10, names
+    for name in names:
+        in_loop = False
+        for line in asm[asm.index(name + ":"):].split(".Lfunc_end", 1)[0].split("\n"):
+            if re.match(r"^\.LBB\S+:", line.strip()):
+                in_loop = "Loop" in line
+            elif in_loop:
+                assert "scratch_" not in line, f"{name}: spill in the tile loop: {line}"

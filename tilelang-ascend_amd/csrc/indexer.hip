@@ -451,10 +451,10 @@ __device__ __forceinline__ void indexer_body(const IdxArgs& a) {
   }
 
   // Stationary q operands and head weights.  fp8: the weights become the A
-  // operands of the head-reduction MFMAs -- every row of A is W (f16), K =
-  // 8g + i standing for head 16*hb0 + 4g + i (i < 4) or 16*hb1 + 4g + i - 4 of
-  // the block pair (hb0, hb1) = (0, 1) or (2, 3), as in relu_operand -- built
-  // with the per-head score scales once q has arrived (fp8_head_scales).
+  // operand of the head-reduction MFMA, built with the per-head score scales once
+  // q has arrived (fp8_head_scales).  Up to 32 heads: every row of A is W (f16),
+  // K = 8g + i standing for head 4g + i (i < 4) or 16 + 4g + i - 4, as in
+  // relu_operand; more: the structured-sparse operand of sparse_sum.
   constexpr bool kMfmaSum = kKind == kFp8;
   constexpr bool kSparseSum = kMfmaSum && kNhb > 2;
   static_assert(!kSparseSum || kTokPW <= 2, "two tokens' rows in one accumulator");
