@@ -216,3 +216,20 @@ def test_up_to_64_heads_tile_and_stage_edges(dsa, dev, B, S, H, topk, paged, dty
     out, lse = dsa.sparse_mla_fwd(q.to(dev), (pool if paged else kv).to(dev), idx.to(dev), 1 / math.sqrt(576), **kw)
     kv[:, 0] = 0
     _check(out, lse, *ref.sparse_mla_fwd(q, kv, want_idx, 1 / math.sqrt(576)))
+
+
+@pytest.mark.parametrize("H,S,paged", [(16, 300, False), (48, 20, True), (64, 260, True)])
+@pytest.mark.parametrize("jump", [40.0, 200.0])
+def test_up_to_64_heads_large_score_jumps(dsa, dev, jump, H, S, paged):
+    """The 64-head kernel's headroom and its exact fallback, whose slot table is made after the loop."""
+    q, kv, idx = _ramp_inputs(jump, H=H, S=S)
+    src, kw = kv, {}
+    if paged:
+        table = torch.randperm(16, generator=torch.Generator().manual_seed(S)).view(1, 16).to(torch.int32)
+        src = torch.empty(16, 64, 1, 576, dtype=kv.dtype)
+        src[table[0].long()] = kv.view(16, 64, 1, 576)
+        kw = dict(block_table=table.to(dev))
+    out, lse = dsa.sparse_mla_fwd(q.to(dev), src.to(dev), idx.to(dev), **kw)
+    ro, rl = ref.sparse_mla_fwd(q, kv, idx)
+    torch.testing.assert_close(out.float().cpu(), ro, atol=2e-2, rtol=2e-2)
+    torch.testing.assert_close(lse.cpu(), rl, atol=1e-3, rtol=1e-3)
