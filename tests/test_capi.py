@@ -71,6 +71,23 @@ def test_python_layer_refuses_cpu_tensors(dsa):
         dsa.sparse_mla_fwd(q, kv, idx)
 
 
+@pytest.mark.parametrize("big", [2**63, -2**63 - 1, 2**70])
+def test_integers_past_64_bits_are_refused_by_the_wrapper(dsa, big):
+    """The native host path leaves them to the wrapper, which names what it refuses."""
+    with pytest.raises(ValueError):
+        dsa.topk_selector(torch.randn(4, 64), big)
+    q, k, w = torch.zeros(1, 2, 4, 64), torch.zeros(1, 8, 1, 64), torch.zeros(1, 2, 4)
+    for change in (dict(sparse_count=big), dict(sparse_mode=big)):
+        with pytest.raises(ValueError):
+            dsa.lightning_indexer(q, k, w, **change)
+    ints = torch.zeros(2, dtype=torch.int32)
+    v4 = dict(ori_kv=torch.zeros(1, 16, 1, 512), ori_block_table=ints[:1].view(1, 1), cu_seqlens_q=ints,
+              seqused_kv=ints[:1], sinks=torch.zeros(16), softmax_scale=0.05)
+    for change in (dict(ori_win_left=big), dict(cmp_ratio=big)):
+        with pytest.raises(ValueError):
+            dsa.sparse_flash_mla(torch.zeros(1, 16, 512), **v4, **change)
+
+
 def test_grouped_sparse_attention_host_logic(dsa):
     """dsa_sparse_attention_fwd: workspace sizes and argument checks (host only)."""
     lib = dsa.load_library()

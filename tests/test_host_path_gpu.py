@@ -135,7 +135,10 @@ def test_plain_arguments(dsa, dev, monkeypatch, name):
     ("indexer_packed", dict(actual_seq_lengths_key=[600, 1401])), ("indexer_packed", dict(block_n=64)),
     ("v4_swa", dict(cu_seqlens_q=[0, 3, 8])), ("v4_swa", dict(cu_seqlens_q=[0, 4, 3])), ("v4_swa", dict(sinks=None)),
     ("v4_hca", dict(cmp_ratio=None)), ("v4_csa", dict(cmp_ratio=None)), ("v4_csa", dict(topk_cmp=4)),
-    ("v4_csa", dict(ori_win_left=-1)), ("v4_swa", dict(return_softmax_lse=False)), ("v4_swa", dict(softmax_scale=1))])
+    ("v4_csa", dict(ori_win_left=-1)), ("v4_swa", dict(return_softmax_lse=False)), ("v4_swa", dict(softmax_scale=1)),
+    ("topk", dict(top_k=2**64 + 100)), ("topk", dict(top_k=-2**70)), ("indexer", dict(sparse_count=2**64 + 200)),
+    ("indexer", dict(sparse_mode=2**32 + 3)), ("indexer_packed", dict(sparse_mode=2**64)),
+    ("v4_swa", dict(ori_win_left=2**64 + 127)), ("v4_csa", dict(cmp_ratio=2**64 + 4))])
 @pytest.mark.parametrize("on_device", [True, False])
 def test_other_arguments(dsa, dev, monkeypatch, name, change, on_device):
     """Refused calls raise the same exception, odd ones give the same result; lengths as device tensors

@@ -68,7 +68,13 @@ struct Arg {
   const T* ptr() const { return t ? static_cast<const T*>(t->data_ptr()) : nullptr; }
 };
 
-int64_t int_of(PyObject* o) { return PyLong_AsLongLong(o); }
+// An exact int that fits 64 bits.
+bool int_of(PyObject* o, int64_t& v) {
+  if (!PyLong_CheckExact(o)) return false;
+  int overflow = 0;
+  v = PyLong_AsLongLongAndOverflow(o, &overflow);
+  return overflow == 0;
+}
 
 // Contiguous, on `dev`, of dtype `st`.
 bool plain(const at::Tensor& t, c10::Device dev, at::ScalarType st) {
@@ -116,11 +122,11 @@ std::vector<int32_t> host_values(const at::Tensor& t) {
 // (x, top_k, sorted, row_len, return_values)
 PyObject* topk(PyObject*, PyObject* const* v, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  DSA_PLAIN(bound && n == 5 && THPVariable_CheckExact(v[0]) && PyLong_CheckExact(v[1]) && PyBool_Check(v[2]) &&
+  int64_t k = 0;
+  DSA_PLAIN(bound && n == 5 && THPVariable_CheckExact(v[0]) && int_of(v[1], k) && PyBool_Check(v[2]) &&
             PyBool_Check(v[4]));
   const at::Tensor& x = THPVariable_Unpack(v[0]);
   const Arg len(v[3]);
-  const int64_t k = int_of(v[1]);
   DSA_PLAIN(x.is_cuda() && x.dim() >= 1 && x.numel() > 0 && plain(x, x.device(), at::kFloat) && k >= 1 && k <= 8192);
   const c10::Device dev = x.device();
   const int64_t cols = x.size(-1), rows = x.numel() / cols;
@@ -147,9 +153,9 @@ PyObject* topk(PyObject*, PyObject* const* v, Py_ssize_t n) {
 // (x, round_scale, out kind)
 PyObject* act_quant(PyObject*, PyObject* const* v, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  DSA_PLAIN(bound && n == 3 && THPVariable_CheckExact(v[0]) && PyBool_Check(v[1]) && PyLong_CheckExact(v[2]));
+  int64_t out = 0;
+  DSA_PLAIN(bound && n == 3 && THPVariable_CheckExact(v[0]) && PyBool_Check(v[1]) && int_of(v[2], out));
   const at::Tensor& x = THPVariable_Unpack(v[0]);
-  const int out = (int)int_of(v[2]);
   const int in = x.scalar_type() == at::kFloat ? DSA_KIND_FP32 : kind16(x.scalar_type());
   DSA_PLAIN(x.is_cuda() && in >= 0 && (x.dim() == 2 || x.dim() == 3) && x.is_contiguous() && x.numel() > 0);
   DSA_PLAIN(out == DSA_KIND_INT8 || out == DSA_KIND_FP8_E4M3);
@@ -163,7 +169,8 @@ PyObject* act_quant(PyObject*, PyObject* const* v, Py_ssize_t n) {
     y = make(sizes, out == DSA_KIND_INT8 ? at::kChar : at::kFloat8_e4m3fn, x.device());
     sizes.back() = 1;
     s = make(sizes, at::kFloat, x.device());
-    rc = E.act_quant(in, x.data_ptr(), rows, cols, out, y.data_ptr(), s.data_ptr<float>(), round, stream(x.device()));
+    rc = E.act_quant(in, x.data_ptr(), rows, cols, (int)out, y.data_ptr(), s.data_ptr<float>(), round,
+                     stream(x.device()));
   }
   DSA_RC(rc);
   return pair(std::move(y), std::move(s));
@@ -301,13 +308,12 @@ PyObject* idx_result(at::Tensor idx, at::Tensor val, bool values, at::ScalarType
 //  key_scale, fuse_topk); packed: TND queries, lengths as prefix sums (keys too, unless paged)
 PyObject* indexer(PyObject*, PyObject* const* v, Py_ssize_t n) {
   HANDLE_TH_ERRORS
+  int64_t K = 0, mode = 0;
   DSA_PLAIN(bound && n == 12 && THPVariable_CheckExact(v[0]) && THPVariable_CheckExact(v[1]) &&
-            THPVariable_CheckExact(v[2]) && PyLong_CheckExact(v[7]) && PyLong_CheckExact(v[8]) && PyBool_Check(v[9]));
+            THPVariable_CheckExact(v[2]) && int_of(v[7], K) && int_of(v[8], mode) && PyBool_Check(v[9]));
   const at::Tensor &q = THPVariable_Unpack(v[0]), &k = THPVariable_Unpack(v[1]), &w = THPVariable_Unpack(v[2]);
   const Arg aq(v[3]), ak(v[4]), bt(v[5]), ks(v[10]);
   const bool packed = v[6] == Py_True, values = v[9] == Py_True;
-  const int64_t K = int_of(v[7]);
-  const int mode = (int)int_of(v[8]);
   DSA_PLAIN(q.is_cuda() && q.dim() == (packed ? 3 : 4) && !aq.other && !ak.other && !ks.other);
   const c10::Device dev = q.device();
   const at::ScalarType st = q.scalar_type();
@@ -379,11 +385,11 @@ PyObject* indexer(PyObject*, PyObject* const* v, Py_ssize_t n) {
     if (packed) {
       rc = (f ? E.tndf : E.tnd)(kind, q.data_ptr(), k.data_ptr(), ks.ptr<float>(), w.data_ptr<float>(), B, rows, S1, S2,
                                 H, D, aq.ptr<int32_t>(), bt ? nullptr : ak.ptr<int32_t>(),
-                                bt ? ak.ptr<int32_t>() : nullptr, bt.ptr<int32_t>(), bs, mb, mode, K,
+                                bt ? ak.ptr<int32_t>() : nullptr, bt.ptr<int32_t>(), bs, mb, (int)mode, K,
                                 idx.data_ptr<int32_t>(), vp, ws.data_ptr(), bytes, stream(dev));
     } else {
       rc = (f ? E.idxf : E.idx)(kind, q.data_ptr(), k.data_ptr(), ks.ptr<float>(), w.data_ptr<float>(), B, S1, S2, H, D,
-                                aq.ptr<int32_t>(), ak.ptr<int32_t>(), bt.ptr<int32_t>(), bs, mb, mode, K,
+                                aq.ptr<int32_t>(), ak.ptr<int32_t>(), bt.ptr<int32_t>(), bs, mb, (int)mode, K,
                                 idx.data_ptr<int32_t>(), vp, ws.data_ptr(), bytes, stream(dev));
     }
   }
@@ -396,8 +402,10 @@ PyObject* indexer(PyObject*, PyObject* const* v, Py_ssize_t n) {
 //  softmax_scale, cmp_ratio, ori_win_left, return lse): packed (TND) queries
 PyObject* flash_mla(PyObject*, PyObject* const* v, Py_ssize_t n) {
   HANDLE_TH_ERRORS
+  int64_t win = 0, ratio = 4;
   DSA_PLAIN(bound && n == 13 && THPVariable_CheckExact(v[0]) && THPVariable_CheckExact(v[1]) &&
-            PyFloat_CheckExact(v[9]) && PyLong_CheckExact(v[11]) && PyBool_Check(v[12]));
+            PyFloat_CheckExact(v[9]) && (v[10] == Py_None || int_of(v[10], ratio)) && int_of(v[11], win) &&
+            PyBool_Check(v[12]));
   const at::Tensor &q = THPVariable_Unpack(v[0]), &ori = THPVariable_Unpack(v[1]);
   const Arg cmp(v[2]), sel(v[3]), obt(v[4]), cbt(v[5]), cu(v[6]), kvl(v[7]), sinks(v[8]);
   DSA_PLAIN(q.is_cuda() && q.dim() == 3 && ori.dim() == 4 && cu && kvl && obt && !cmp.other && !sel.other &&
@@ -405,17 +413,13 @@ PyObject* flash_mla(PyObject*, PyObject* const* v, Py_ssize_t n) {
   const c10::Device dev = q.device();
   const at::ScalarType st = q.scalar_type();
   const int kind = kind16(st);
-  const int64_t T = q.size(0), H = q.size(1), B = cu.t->numel() - 1, win = int_of(v[11]);
+  const int64_t T = q.size(0), H = q.size(1), B = cu.t->numel() - 1;
   DSA_PLAIN(kind >= 0 && plain(q, dev, st) && plain(ori, dev, st) && T > 0 && H >= 16 && H % 16 == 0 && H <= 1024 &&
             q.size(2) == 512 && ori.size(2) == 1 && ori.size(3) == 512 && B >= 1 && cu.t->dim() == 1 &&
             plain(*cu.t, dev, at::kInt) && plain(*kvl.t, dev, at::kInt) && kvl.t->numel() == B &&
             table_ok(obt, dev, B));
   if (sinks) DSA_PLAIN(plain(*sinks.t, dev, at::kFloat) && sinks.t->numel() == H);
-  int64_t K = 0, ratio = 4, cmp_blocks = 0, cmp_bs = 0, cmp_tl = 0;
-  if (v[10] != Py_None) {
-    DSA_PLAIN(PyLong_CheckExact(v[10]));
-    ratio = int_of(v[10]);
-  }
+  int64_t K = 0, cmp_blocks = 0, cmp_bs = 0, cmp_tl = 0;
   if (cmp) {
     DSA_PLAIN(cmp.t->dim() == 4 && plain(*cmp.t, dev, st) && cmp.t->size(2) == 1 && cmp.t->size(3) == 512 && cbt &&
               table_ok(cbt, dev, B) && ratio >= 1 && (sel || v[10] != Py_None));
