@@ -134,6 +134,21 @@ def test_decode_rows_masked_slots(dsa, dev, dtype):
         assert torch.count_nonzero(out[0, 1]) == 0
 
 
+@pytest.mark.parametrize("m,topk", [(1, 150), (3, 150), (4, 1000)])
+def test_decode_rows_read_no_key_for_empty_slots(dsa, dev, m, topk):
+    """At most 8 query rows: key 0 is NaN and never selected; -1 slots and those past the list's end
+    must not bring it in."""
+    print(f"sparse_attn decode rows, NaN in key 0: b=2 m={m} topk={topk}", flush=True)
+    q, kv, sink, idx = _inputs(2, m, 300, 32, 512, topk, torch.bfloat16, 48)
+    idx = idx.clamp(min=1)
+    idx[:, :, ::3] = -1
+    idx[1, 0, 16:32] = -1
+    want, want_lse = ref.sparse_attn_sink(q, kv, sink, idx, 0.05)
+    kv[0, 0] = float("nan")
+    _check_out(_run(dsa, dev, q, kv, sink, idx, 0.05), want, torch.bfloat16)
+    torch.testing.assert_close(_lse(dsa, dev, q, kv, sink, idx, 0.05), want_lse, rtol=1e-3, atol=1e-3)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_decode_rows_chunked(dsa, dev, dtype):
     """At most 8 query rows with 257..1024 slots: the decode kernel in 128-slot chunks whose

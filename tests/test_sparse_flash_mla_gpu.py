@@ -295,3 +295,27 @@ def test_decode_rows_many_batches(dsa, dev):
                     win_left=win)
     wo, wl = _want(q, cu, kv_lens, ori, ori_bt, sinks, 0.05, cmp=cmp, cmp_bt=cmp_bt, ratio=ratio, win_left=win)
     _check(out, lse, wo, wl, torch.bfloat16)
+
+
+@pytest.mark.parametrize("scenario", ["swa", "hca", "csa"])
+def test_decode_rows_read_no_cache_row_for_empty_slots(dsa, dev, scenario):
+    """Up to 8 rows: block 0 of the window's cache holds NaN and is in no table; slots past the list's
+    end (and csa's skipped entries) must not bring it in."""
+    H, K, bs, ratio, win = 32, 300, 16, 4, 40
+    cu, kv_lens = [0, 1, 4], [700, 333]
+    g = torch.Generator().manual_seed(17)
+    q = torch.randn((cu[-1], H, 512), generator=g).to(torch.bfloat16)
+    ori, ori_bt = _paged(kv_lens, bs, 70, 512, -1, 1, torch.bfloat16, g)
+    ori = torch.cat((torch.full((1, bs, 1, 512), float("nan"), dtype=ori.dtype), ori))
+    ori_bt = torch.where(ori_bt >= 0, ori_bt + 1, ori_bt)
+    cmp = cmp_bt = idx = None
+    if scenario != "swa":
+        cmp, cmp_bt = _paged([n // ratio for n in kv_lens], bs, 20, 512, -1, 1, torch.bfloat16, g)
+    if scenario == "csa":
+        idx = _csa_indices(cu, kv_lens, K, ratio, g)
+        idx[:, 0, 20:40] = 5000  # past the threshold: skipped
+    r = ratio if scenario != "swa" else None
+    args = (cu, kv_lens, ori, ori_bt, torch.randn(H, generator=g), 0.05)
+    out, lse = _run(dsa, dev, q, *args, cmp=cmp, cmp_bt=cmp_bt, idx=idx, ratio=r, win_left=win)
+    wo, wl = _want(q, *args, cmp=cmp, cmp_bt=cmp_bt, idx=idx, ratio=r, win_left=win)
+    _check(out, lse, wo, wl, torch.bfloat16)

@@ -233,3 +233,40 @@ def test_up_to_64_heads_large_score_jumps(dsa, dev, jump, H, S, paged):
     ro, rl = ref.sparse_mla_fwd(q, kv, idx)
     torch.testing.assert_close(out.float().cpu(), ro, atol=2e-2, rtol=2e-2)
     torch.testing.assert_close(lse.cpu(), rl, atol=1e-3, rtol=1e-3)
+
+
+@pytest.mark.parametrize("T", [1, 2, 8])
+@pytest.mark.parametrize("topk", [40, 300])  # one workgroup per row and 16 heads / chunks
+@pytest.mark.parametrize("form", ["contiguous", "paged", "parts", "parts_paged"])
+def test_decode_rows_read_no_key_for_empty_slots(dsa, dev, T, topk, form):
+    """Up to 8 rows: the cache's first row is NaN and never selected; -1 slots, slots past the causal
+    bound or the end of the list, and blocks without a valid slot must not bring it in."""
+    g = torch.Generator().manual_seed(100 * T + topk)
+    H, skv, bs, dt = 32, 640, 64, torch.bfloat16
+    apart = form.startswith("parts")
+    B, S = (1, T) if apart else (T, 1)
+    q = (torch.randn(B, S, H, 576, generator=g) * 0.5).to(dt)
+    kv = (torch.randn(B, skv, 1, 576, generator=g) * 0.5).to(dt)
+    idx = torch.stack([1 + torch.randperm(skv - 1, generator=g)[:topk] for _ in range(B * S)]).to(torch.int32)
+    idx[:, ::3] = -1
+    idx[:, 16:33] = -1                                   # a whole block, then past the key length
+    idx = idx.view(B, S, 1, topk)
+    kl = torch.tensor([skv - 40] * B, dtype=torch.int32)
+    want, want_lse = ref.sparse_mla_fwd(q, kv, idx, 0.05, actual_seq_lengths_kv=kl.tolist())
+    kv[0, 0] = float("nan")
+    src, kw = kv, {}
+    if form.endswith("paged"):
+        n = skv // bs
+        perm = 1 + torch.randperm(B * n, generator=g)
+        src = torch.full((B * n + 1, bs, 1, 576), float("nan"), dtype=dt)  # block 0 holds no key
+        src[perm] = kv.view(B * n, bs, 1, 576)
+        kw = dict(block_table=perm.view(B, n).to(torch.int32).to(dev))
+    if apart:
+        cut = lambda t: (t[..., :512].contiguous().to(dev), t[..., 512:].contiguous().to(dev))  # noqa: E731
+        (ql, qr), (kc, kr) = cut(q[0]), cut(src)
+        out = dsa.sparse_attn_tilelang(ql, kc, kc, idx[0].to(dev), 0.05, 1, None, kl.to(dev), query_rope=qr, key_rope=kr,
+                                       sparse_mode=3, **kw)
+        torch.testing.assert_close(out[None].float().cpu(), want, atol=2e-2, rtol=2e-2)
+    else:
+        out, lse = dsa.sparse_mla_fwd(q.to(dev), src.to(dev), idx.to(dev), 0.05, actual_seq_lengths_kv=kl.to(dev), **kw)
+        _check(out, lse, want, want_lse)

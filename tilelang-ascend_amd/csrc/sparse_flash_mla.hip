@@ -306,6 +306,9 @@ __device__ __forceinline__ short dec_round(float p, float& back) {
   }
 }
 
+// Empty slots load this row: probability 0 times a NaN or infinity of any cache row would not be 0.
+static __device__ __align__(128) uint8_t kDecZeroRow[576 * 2];
+
 // kMode: 0 row lists given (rows / count), 1 swa, 2 hca, 3 csa (lists derived
 // here), 4 sparse MLA index rows (kD = 576: K is the whole row, V its first 512).
 template <bool kF16, int kMode, int kD = 512>
@@ -489,6 +492,8 @@ __global__ __launch_bounds__(256) void v4_decode_rows_kernel(DecArgs a) {
   uint8_t* wbuf = lds + wave * (2 * kBlkLds);
   const int s_hi = min(cnt, s_lo + a.chunk);
   const int nblk = s_hi > s_lo ? (s_hi - s_lo + kDecBlk - 1) / kDecBlk : 0;
+  const uint8_t* zero_row = kDecZeroRow;
+  __asm__("" : "+s"(zero_row));  // the address is kept, not looked up again for each block
   // DMA of the wave's block i to bp; returns its valid-slot mask.  rowg[0] holds
   // block i's group: the groups shift down when block i starts one.
   auto load = [&](int i, uint8_t* bp) -> uint32_t {
@@ -500,7 +505,7 @@ __global__ __launch_bounds__(256) void v4_decode_rows_kernel(DecArgs a) {
     const int32_t rows = rowg[0];
     const bool valid = rows >= 0 && slot_of(k) < cnt;
     const uint32_t vmask = (uint32_t)(__builtin_amdgcn_ballot_w64(valid) >> (16 * j)) & 0xffffu;
-    const int32_t rz = valid ? rows : 0;  // empty slots read row 0 (their scores are masked)
+    const int32_t rz = valid ? rows : -1;  // empty slots read zero_row
     constexpr int kRowBytes = kTails ? 1024 : kD * 2;
 #pragma unroll
     for (int u = 0; u < kDecBlk; ++u) {
@@ -508,7 +513,7 @@ __global__ __launch_bounds__(256) void v4_decode_rows_kernel(DecArgs a) {
       // Index rows (kMla) use all 31 bits; V4 lists tag compressed rows.
       const uint8_t* base = (!kMla && (ru & kCmpTag)) ? a.kv2 : a.kv;
       const int64_t pr = kMla ? (int64_t)ru : (int64_t)(ru & ~kCmpTag);
-      const uint8_t* src = base + pr * kRowBytes + 16 * (lane ^ (2 * u));
+      const uint8_t* src = (ru < 0 ? zero_row : base + pr * kRowBytes) + 16 * (lane ^ (2 * u));
       __builtin_amdgcn_global_load_lds((dec_gbl_void*)src, (dec_lds_void*)(bp + u * 1024), 16, 0, 0);
     }
     if constexpr (kD == 576) {
@@ -520,7 +525,8 @@ __global__ __launch_bounds__(256) void v4_decode_rows_kernel(DecArgs a) {
         const int ruq = __shfl(rz, 16 * j + 8 * q + (lane >> 3), kWave);
         const int u = 8 * q + (lane >> 3);
         const int c = (lane & 7) ^ (2 * ((u >> 2) & 3));
-        const uint8_t* src = (kTails ? a.kv2 + (int64_t)ruq * 128 : a.kv + (int64_t)ruq * kRowBytes + 1024) + 16 * c;
+        const uint8_t* tail = kTails ? a.kv2 + (int64_t)ruq * 128 : a.kv + (int64_t)ruq * kRowBytes + 1024;
+        const uint8_t* src = (ruq < 0 ? zero_row : tail) + 16 * c;
         __builtin_amdgcn_global_load_lds((dec_gbl_void*)src, (dec_lds_void*)(bp + kDecBlk * 1024 + q * 1024), 16, 0, 0);
       }
     }
