@@ -136,6 +136,26 @@ def test_gqa_ragged_and_max_topk(dsa, dev, topk):
     _check(out, lse, ro, rl, torch.float16)
 
 
+@pytest.mark.parametrize("G,Hg", [(2, 16), (1, 40)])
+@pytest.mark.parametrize("topk", [33, 500])
+def test_gqa_reads_no_key_for_empty_slots(dsa, dev, G, Hg, topk):
+    """Key 0 is NaN and never selected; -1 slots, slots past the causal bound and past the list's end
+    must not bring it in."""
+    B, S, Skv = 2, 9, 700
+    g = torch.Generator().manual_seed(topk + G)
+    q = torch.randn(B, S, G * Hg, 128, generator=g).to(torch.bfloat16)
+    kv = torch.randn(B, Skv, G, 128, generator=g).to(torch.bfloat16)
+    idx = _grouped_indices(B, S, G, Skv, topk, seed=topk)
+    idx = torch.where(idx == 0, torch.full_like(idx, -1), idx)
+    idx[:, 1, :, :32] = -1  # the first tile empty
+    idx[1, 2] = -1          # no valid slot
+    _log(f"GQA, NaN in key 0: G={G} Hg={Hg} topk={topk}")
+    ro, rl = ref.sparse_attention_grouped(q, kv, idx, d_v=128)
+    kv[:, 0] = float("nan")
+    out, lse = dsa.sparse_gqa_fwd(q.to(dev), kv.to(dev), idx.to(dev))
+    _check(out, lse, ro, rl, torch.bfloat16)
+
+
 def _mla_group_inputs(B, S, Skv, G, Hg, topk, seed, dtype=torch.bfloat16):
     g = torch.Generator().manual_seed(seed)
     q = (torch.randn(B, S, G * Hg, 576, generator=g) * 0.5).to(dtype)

@@ -27,6 +27,8 @@
 // (each lane holds 8 scores of one head), and O^T += V^T P^T (8 blocks of 16
 // output columns, V^T through ds_read_b64_tr_b16).  Each slot brings 256 bytes
 // for 16 x 2 x 2 x 128 flops per 16 heads: the loop is bound by the gather.
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace dsa {
@@ -128,6 +130,9 @@ __host__ __device__ constexpr int gqa_lds_bytes(int stg, int hb, int ntiles) {
   return gqa_ring_bytes(stg) + ntiles * kGqaTile * 4 + ntiles * 4 + (ntiles + 1) * 4 + kGqaWaves * 16 * hb * 2 * 4;
 }
 
+// Empty slots load this row: probability 0 times a NaN or infinity of any KV row would not be 0.
+static __device__ __align__(128) uint8_t kGqaZeroRow[kGqaRowBytes];
+
 template <bool kF16, int kHB, int kStg>
 __global__ __launch_bounds__(kGqaThreads, 2) void sparse_gqa_kernel(GqaArgs a) {
   static_assert(kStg >= 2 && kStg <= 3, "ring depth: the merge reuses a wave's ring (16 KB per 16 heads x 2)");
@@ -223,10 +228,10 @@ __global__ __launch_bounds__(kGqaThreads, 2) void sparse_gqa_kernel(GqaArgs a) {
   uint8_t* ring = lds + wave * kStg * kGqaTileBytes;
   const uint8_t* kvb = reinterpret_cast<const uint8_t*>(a.kv);
   const int q4 = lane >> 4;
+  const uint8_t* zero_row = kGqaZeroRow;
+  __asm__("" : "+s"(zero_row));  // the address is kept, not looked up again for each tile
   // DMA of entry e into stage st: instruction n moves keys 4n .. 4n + 3; lane l
-  // fetches chunk (l & 15) ^ gqa_swz(4n + q4) of key 4n + q4.  Tiles in the list
-  // hold a valid slot, so kv_len >= 1 and row0 (idx 0) is a row of the cache:
-  // empty slots load it and get probability 0.
+  // fetches chunk (l & 15) ^ gqa_swz(4n + q4) of key 4n + q4 (empty slots: of zero_row).
   auto dma = [&](int e, int st) {
     const int tile = __builtin_amdgcn_readlane(my_tile, e);
     const uint32_t taddr = gqa_lds_u32(rows + tile * kGqaTile + 8 * q4);
@@ -235,13 +240,19 @@ __global__ __launch_bounds__(kGqaThreads, 2) void sparse_gqa_kernel(GqaArgs a) {
     gqa_b128<16>(rv[1], taddr);
     gqa_lgkm_wait(rv);
     uint8_t* dst = ring + st * kGqaTileBytes;
+    const auto issue = [&](auto full) {
 #pragma unroll
-    for (int n = 0; n < 8; ++n) {
-      int rw = (int)rv[n / 4][n % 4];
-      rw = rw >= 0 ? rw : row0;
-      const uint8_t* src = kvb + (int64_t)rw * kGqaRowBytes + 16 * ((lane & 15) ^ gqa_swz(4 * n + q4));
-      __builtin_amdgcn_global_load_lds((gqa_gbl_void*)src, (gqa_lds_void*)(dst + n * 1024), 16, 0, 0);
-    }
+      for (int n = 0; n < 8; ++n) {
+        const int rw = (int)rv[n / 4][n % 4];
+        const uint8_t* p = kvb + (int64_t)rw * kGqaRowBytes;
+        const uint8_t* src = (full || rw >= 0 ? p : zero_row) + 16 * ((lane & 15) ^ gqa_swz(4 * n + q4));
+        __builtin_amdgcn_global_load_lds((gqa_gbl_void*)src, (gqa_lds_void*)(dst + n * 1024), 16, 0, 0);
+      }
+    };
+    // Tiles without an empty slot, most of them, choose no address (with a choice in
+    // every tile 546 rows of 64 heads over 4 and 2048 slots took 128.2 us, 126.3 without).
+    if (__builtin_amdgcn_readlane((int)my_mask, e) == -1) issue(std::true_type{});
+    else issue(std::false_type{});
   };
 
   // Operand offsets in a stage.  K (A of S^T = K Q^T, step st, key block kb):
