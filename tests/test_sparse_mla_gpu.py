@@ -184,16 +184,28 @@ def test_large_score_jumps(dsa, dev, jump, S):
     torch.testing.assert_close(lse.cpu(), rl, atol=1e-3, rtol=1e-3)
 
 
-@pytest.mark.parametrize("B,S,H,topk,paged", [(1, 9, 16, 31, False), (3, 3, 48, 1100, True), (2, 130, 64, 33, True),
-                                              (120, 1, 32, 1100, True), (1, 120, 64, 1088, False),
-                                              (1, 300, 48, 2049, False)])
+def _ring_depth(dsa, B, S, H, topk):
+    """Stages the 64-head kernel's launch picks: 3 where the grid has at most 256 workgroups of more
+    than 512 slots each.  The split count is read off the workspace (split partials of 512 16-bit
+    values and an fp32 LSE per row and head, and 256 bytes)."""
+    ws = dsa.load_library().dsa_sparse_mla_workspace_size(B, S, H, topk)
+    splits = (ws - 256) // (B * S * H * (512 * 2 + 4)) if ws else 1
+    per = math.ceil(math.ceil(topk / splits) / 32) * 32
+    return 3 if B * S * splits <= 256 and per > 512 else 2
+
+
+@pytest.mark.parametrize("B,S,H,topk,paged,stages", [
+    (1, 9, 16, 31, False, 2), (3, 3, 48, 1100, True, 2), (2, 130, 64, 33, True, 2), (120, 1, 32, 1100, True, 2),
+    (1, 120, 64, 1088, False, 2), (1, 300, 48, 2049, False, 2), (1, 128, 64, 2048, False, 3), (2, 64, 16, 2048, True, 3),
+    (1, 256, 48, 1100, False, 3), (2, 128, 64, 545, True, 3)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_up_to_64_heads_tile_and_stage_edges(dsa, dev, B, S, H, topk, paged, dtype):
+def test_up_to_64_heads_tile_and_stage_edges(dsa, dev, B, S, H, topk, paged, stages, dtype):
     """The 64-head kernel: both ring depths, splits, ragged last tiles, empty tiles, heads short of 64.
 
     Slots are emptied by -1 and, in a paged cache, by a block of a negative number; key 0 is NaN and
     never selected, so an empty slot that reads a key instead of zeros shows.
     """
+    assert _ring_depth(dsa, B, S, H, topk) == stages
     g = torch.Generator().manual_seed(B * S + H + topk)
     skv, bs = 2112, 64
     q = (torch.randn(B, S, H, 576, generator=g) * 0.5).to(dtype)
@@ -218,16 +230,20 @@ def test_up_to_64_heads_tile_and_stage_edges(dsa, dev, B, S, H, topk, paged, dty
     _check(out, lse, *ref.sparse_mla_fwd(q, kv, want_idx, 1 / math.sqrt(576)))
 
 
-@pytest.mark.parametrize("H,S,paged", [(16, 300, False), (48, 20, True), (64, 260, True)])
+@pytest.mark.parametrize("H,S,paged,topk", [(16, 300, False, 256), (48, 20, True, 256), (64, 260, True, 256),
+                                            (64, 256, True, 1000), (16, 256, False, 1000)])
 @pytest.mark.parametrize("jump", [40.0, 200.0])
-def test_up_to_64_heads_large_score_jumps(dsa, dev, jump, H, S, paged):
-    """The 64-head kernel's headroom and its exact fallback, whose slot table is made after the loop."""
-    q, kv, idx = _ramp_inputs(jump, H=H, S=S)
+def test_up_to_64_heads_large_score_jumps(dsa, dev, jump, H, S, paged, topk):
+    """The 64-head kernel's headroom and its exact fallback, whose slot table is made after the loop
+    (topk 1000: from three stages)."""
+    assert _ring_depth(dsa, 1, S, H, topk) == (3 if topk == 1000 else 2)
+    q, kv, idx = _ramp_inputs(jump, H=H, S=S, topk=topk, Skv=2048 if topk == 1000 else 1024)
     src, kw = kv, {}
     if paged:
-        table = torch.randperm(16, generator=torch.Generator().manual_seed(S)).view(1, 16).to(torch.int32)
-        src = torch.empty(16, 64, 1, 576, dtype=kv.dtype)
-        src[table[0].long()] = kv.view(16, 64, 1, 576)
+        n = kv.shape[1] // 64
+        table = torch.randperm(n, generator=torch.Generator().manual_seed(S)).view(1, n).to(torch.int32)
+        src = torch.empty(n, 64, 1, 576, dtype=kv.dtype)
+        src[table[0].long()] = kv.view(n, 64, 1, 576)
         kw = dict(block_table=table.to(dev))
     out, lse = dsa.sparse_mla_fwd(q.to(dev), src.to(dev), idx.to(dev), **kw)
     ro, rl = ref.sparse_mla_fwd(q, kv, idx)

@@ -1398,8 +1398,7 @@ void sparse_mla_rows4_kernel(MlaArgs a) {
 // 4000 rows of 8000 keys at 16 / 48 / 64 heads 1776 -> 1070, 1690 -> 1075,
 // 1705 -> 1090; 64 decode rows at 16 / 64 heads 51 -> 41, 53 -> 48; 400 rows at
 // 64 heads 236 -> 192.
-// kStages: 3 where a grid has one workgroup per CU anyway and long rows (two tiles
-// in flight; 128 rows at 64 heads 84 -> 76 us, at 16 heads 75 -> 65), else 2.
+// kStages: 3 (two tiles in flight) or 2, as launch_mla_heads64 picks.
 template <int kStages>
 struct H64Lds {
   static constexpr int kMaskOffset = kStages * MlaGeom<576>::kStageBytes + kR4PBytes;
@@ -1919,8 +1918,14 @@ static hipError_t launch_mla_heads64(const MlaArgs& a, hipStream_t stream) {
   const auto paged = [&](auto stages) {
     return a.block_table ? launch(std::true_type{}, stages) : launch(std::false_type{}, stages);
   };
-  // One workgroup per CU at most: the third stage is free, and pays past 16 tiles a
-  // workgroup (at 4 or 16 tiles both take the same time, within 1 us).
+  // A grid of at most one workgroup per CU has the LDS for a third stage.  Splits
+  // double until they make 256 workgroups, so with more than 16 tiles each this is
+  // exactly 256: batches of 64 rows (past 2048 slots), 128 (past 1024) and 256.
+  // Decode batches over paged caches of 64K (256 rows: 32K) tokens each, two -> three
+  // stages, 2048 slots: 128 rows at 64 / 16 heads 79 -> 72, 68 -> 63 us, 256 rows
+  // 139 -> 128, 130 -> 121; 1024 slots, 256 rows 73 -> 66; at 64 rows of 2100 slots,
+  // 128 of 1100 and 256 of 600 no difference; rows that share one cache of 32768 keys
+  // (gathered out of the MALL) within 2 us either way.
   return wgs <= 256 && a.keys_per_split > 16 * kMlaTile ? paged(std::integral_constant<int, 3>{})
                                                         : paged(std::integral_constant<int, 2>{});
 }
