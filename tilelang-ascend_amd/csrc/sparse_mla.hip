@@ -53,6 +53,7 @@ constexpr int kMlaDV = 512;
 constexpr int kMlaTile = 32;                       // slots per tile
 constexpr int kStages = 4;
 constexpr int kAhead = kStages - 1;                // tiles in flight ahead of compute
+constexpr int kMlaWaves = 4;                       // waves per workgroup, one row group of a tile's DMA each
 constexpr int kSlotsCap = 2048;                    // slots per workgroup (physical rows kept in LDS)
 // Rows with this bit set live in the second KV source (MlaArgs::kv2).
 constexpr int32_t kSrc2Bit = 0x40000000;
@@ -156,13 +157,12 @@ __device__ __forceinline__ void wait_tiles(int ahead) {
   }
 }
 
-template <int kNW, int kD>
+template <int kD>
 struct MlaCfg {
-  static constexpr int kThreads = kNW * kWave;
+  static constexpr int kThreads = kMlaWaves * kWave;
   static constexpr int kTileInstr = MlaGeom<kD>::kTileInstr;
-  // DMA instructions per tile for wave w: I = w, w + kNW, ... < kTileInstr.
-  static constexpr int kMaxPerWave = (kTileInstr + kNW - 1) / kNW;
-  static_assert(kTileInstr % kNW == 0, "every wave issues the same number of DMA loads per tile");
+  static constexpr int kMaxPerWave = kTileInstr / kMlaWaves;  // DMA instructions per tile and wave
+  static_assert(kTileInstr % kMlaWaves == 0, "every wave issues the same number of DMA loads per tile");
   // Tiles issued ahead of the one being multiplied by P V.  Iteration t needs
   // tile t+1 resident (for its Q K^T) and keeps tiles t+2 .. t+kDepth-1 in
   // flight, so kDepth >= 2; kDepth - 1 tiles of loads must fit the 6-bit vmcnt
@@ -191,59 +191,47 @@ __host__ __device__ constexpr int lds_swizzle(int u, int a) {
 }
 
 // The DMA of tile `tile` (slots tile*32 .. +31 of this workgroup) into a
-// stage.  Wave w fills the row groups a = w, w + kNW, ...; lane 8u + v loads
-// chunk 8b + (v ^ lds_swizzle(u, a)) of slot 8a + u, so its row address is
-// fixed per row group and only the chunk-group offset 128*b changes between
-// instructions.  Empty / masked slots re-load `safe_row` (a valid row of this
-// workgroup; its probability is forced to 0), so every load stays inside the
-// KV cache.
+// stage.  Wave w fills row group a = w; lane 8u + v loads chunk
+// 8b + (v ^ lds_swizzle(u, a)) of slot 8a + u, so its row address is fixed and
+// only the chunk-group offset 128*b changes between instructions.  Empty /
+// masked slots re-load `safe_row` (a valid row of this workgroup; its
+// probability is forced to 0), so every load stays inside the KV cache.
 // The same DMA, split so that its instructions can be spread over the
-// matrix work of an iteration: prepare() computes the lane's row addresses
+// matrix work of an iteration: prepare() computes the lane's row address
 // (reading the slot -> row map from LDS; a row tagged kSrc2Bit is read from
 // the second source), issue<D>() sends instruction D.
 // Sent in one burst, the instructions of the four waves queue behind each
 // other in the memory pipeline and stall the issuing waves.
-template <int kNW, int kD>
+template <int kD>
 struct TileDma {
-  static constexpr int kRowChunks = MlaGeom<kD>::kRowChunks;
-  static constexpr int kGroups = 4 / kNW;                    // row groups per wave
-  static constexpr int kCount = kGroups * (kRowChunks / 8);  // instructions per wave and tile
-  const uint8_t* src[kGroups];
+  static constexpr int kCount = MlaGeom<kD>::kRowChunks / 8;  // instructions per wave and tile
+  const uint8_t* src;
   uint8_t* stage;
   int wave;
 
   __device__ __forceinline__ void prepare(const uint8_t* kv, const uint8_t* kv2, const int32_t* rows, int safe_row,
                                           int tile, uint8_t* stage_base, int wave_, int lane) {
-    wave = wave_;
-    stage = stage_base;
     const int u = lane >> 3;
-#pragma unroll
-    for (int ag = 0; ag < kGroups; ++ag) {
-      const int a = wave + ag * kNW;
-      int row = rows[tile * kMlaTile + 8 * a + u];
-      row = row >= 0 ? row : safe_row;
-      const uint8_t* base = kv;
-      if constexpr (MlaGeom<kD>::kRowLists) {
-        base = (row & kSrc2Bit) ? kv2 : kv;
-        row &= ~kSrc2Bit;
-      }
-      src[ag] = base + (int64_t)row * MlaGeom<kD>::kRowBytes + 16 * ((lane & 7) ^ lds_swizzle(u, a));
+    int row = rows[tile * kMlaTile + 8 * wave_ + u];
+    row = row >= 0 ? row : safe_row;
+    const uint8_t* base = kv;
+    if constexpr (MlaGeom<kD>::kRowLists) {
+      base = (row & kSrc2Bit) ? kv2 : kv;
+      row &= ~kSrc2Bit;
     }
+    prepare_src(base + (int64_t)row * MlaGeom<kD>::kRowBytes + 16 * ((lane & 7) ^ lds_swizzle(u, wave_)), stage_base,
+                wave_);
   }
-  // One row group per wave, the lane's source address given.
+  // The lane's source address given.
   __device__ __forceinline__ void prepare_src(const uint8_t* lane_src, uint8_t* stage_base, int wave_) {
-    static_assert(kGroups == 1, "one row group per wave");
     wave = wave_;
     stage = stage_base;
-    src[0] = lane_src;
+    src = lane_src;
   }
   template <int D>
   __device__ __forceinline__ void issue() {
     static_assert(D >= 0 && D < kCount, "DMA instruction index");
-    constexpr int kAg = D / (kRowChunks / 8), kB = D % (kRowChunks / 8);
-    const int a = wave + kAg * kNW;
-    __builtin_amdgcn_global_load_lds((gbl_void*)(src[kAg] + 128 * kB), (lds_void*)(stage + (a + 4 * kB) * 1024), 16,
-                                     0, 0);
+    __builtin_amdgcn_global_load_lds((gbl_void*)(src + 128 * D), (lds_void*)(stage + (wave + 4 * D) * 1024), 16, 0, 0);
   }
 };
 
@@ -363,20 +351,20 @@ __device__ __forceinline__ void lgkm_wait_k(u32x4& k) {
   __asm__ __volatile__("s_waitcnt lgkmcnt(%1)" : "+v"(k) : "i"(N));
 }
 
-template <int kNW, int kD, int D = 0>
-__device__ __forceinline__ void il_dma_all(TileDma<kNW, kD>& dma) {
-  if constexpr (D < TileDma<kNW, kD>::kCount) {
+template <int kD, int D = 0>
+__device__ __forceinline__ void il_dma_all(TileDma<kD>& dma) {
+  if constexpr (D < TileDma<kD>::kCount) {
     dma.template issue<D>();
-    il_dma_all<kNW, kD, D + 1>(dma);
+    il_dma_all<kD, D + 1>(dma);
   }
 }
 
 // DMA instructions D with D * kQkHalf / kCount == J go out at half-step J.
-template <int kNW, int kD, int J, int D = 0>
-__device__ __forceinline__ void il_dma(TileDma<kNW, kD>& dma) {
-  if constexpr (D < TileDma<kNW, kD>::kCount) {
-    if constexpr (D * MlaGeom<kD>::kQkHalf / TileDma<kNW, kD>::kCount == J) dma.template issue<D>();
-    il_dma<kNW, kD, J, D + 1>(dma);
+template <int kD, int J, int D = 0>
+__device__ __forceinline__ void il_dma(TileDma<kD>& dma) {
+  if constexpr (D < TileDma<kD>::kCount) {
+    if constexpr (D * MlaGeom<kD>::kQkHalf / TileDma<kD>::kCount == J) dma.template issue<D>();
+    il_dma<kD, J, D + 1>(dma);
   }
 }
 
@@ -415,15 +403,15 @@ __device__ __forceinline__ void mfma_qk(f32x4& c, const u32x4& a, const u32x4& b
   }
 }
 
-template <bool kF16, int kNW, int kD, bool kDma, int J>
+template <bool kF16, int kD, bool kDma, int J>
 __device__ __forceinline__ void qk_half(f32x4 (&c)[2][2][2], const u32x4 (&qb)[2][kD / 32],
-                                        const uint32_t (&qa)[2], u32x4 (&k)[kQkAhead + 1], TileDma<kNW, kD>& dma) {
+                                        const uint32_t (&qa)[2], u32x4 (&k)[kQkAhead + 1], TileDma<kD>& dma) {
   constexpr int kQkHalf = MlaGeom<kD>::kQkHalf;
   constexpr int kNext = J + kQkAhead;
   if constexpr (kNext < kQkHalf) {
     b128_read<4096 * (kNext / 4) + 2048 * (kNext % 2)>(k[kNext % (kQkAhead + 1)], qa[(kNext / 2) % 2]);
   }
-  if constexpr (kDma) il_dma<kNW, kD, J>(dma);
+  if constexpr (kDma) il_dma<kD, J>(dma);
   constexpr int kWait = (kQkHalf - 1 - J) < kQkAhead ? (kQkHalf - 1 - J) : kQkAhead;
   constexpr int kSlot = J % (kQkAhead + 1);
   lgkm_wait_k<kWait>(k[kSlot]);
@@ -431,7 +419,7 @@ __device__ __forceinline__ void qk_half(f32x4 (&c)[2][2][2], const u32x4 (&qb)[2
   // Half-steps 0..3 start the four chains of each head block.
   mfma_qk<kF16, (J < 4)>(c[kSet][0][kKb], k[kSlot], qb[0][kSt]);
   mfma_qk<kF16, (J < 4)>(c[kSet][1][kKb], k[kSlot], qb[1][kSt]);
-  if constexpr (J + 1 < kQkHalf) qk_half<kF16, kNW, kD, kDma, J + 1>(c, qb, qa, k, dma);
+  if constexpr (J + 1 < kQkHalf) qk_half<kF16, kD, kDma, J + 1>(c, qb, qa, k, dma);
 }
 
 template <int J>
@@ -442,13 +430,13 @@ __device__ __forceinline__ void qk_prologue(u32x4 (&k)[kQkAhead + 1], const uint
   }
 }
 
-template <bool kF16, int kNW, int kD, bool kDma>
+template <bool kF16, int kD, bool kDma>
 __device__ __forceinline__ void qk_phase(f32x4 (&s)[2][2], const u32x4 (&qb)[2][kD / 32],
-                                         const uint32_t (&qa)[2], TileDma<kNW, kD>& dma) {
+                                         const uint32_t (&qa)[2], TileDma<kD>& dma) {
   f32x4 c[2][2][2];
   u32x4 k[kQkAhead + 1];
   qk_prologue<0>(k, qa);
-  qk_half<kF16, kNW, kD, kDma, 0>(c, qb, qa, k, dma);
+  qk_half<kF16, kD, kDma, 0>(c, qb, qa, k, dma);
   static_assert(kQkAhead + 1 == 7, "the wait below names every K operand register");
   // The asm MFMAs are opaque to the compiler's hazard checks: 24 wait states
   // (a 16-pass MFMA needs 19) before a VALU instruction reads a result, and
@@ -621,9 +609,9 @@ __device__ __attribute__((noinline)) void mla_exact_fallback(const uint16_t* q, 
 }
 
 // kPaged: the KV rows are addressed through a block table (a.block_table).
-template <int kNW, bool kF16, int kD, bool kPaged>
-__global__ __launch_bounds__(kNW * kWave) void sparse_mla_kernel(MlaArgs a) {
-  using Cfg = MlaCfg<kNW, kD>;
+template <bool kF16, int kD, bool kPaged>
+__global__ __launch_bounds__(kMlaWaves * kWave) void sparse_mla_kernel(MlaArgs a) {
+  using Cfg = MlaCfg<kD>;
   using Geo = MlaGeom<kD>;
   using Lay = MlaLayout<kD, kStages>;
   extern __shared__ __align__(16) uint8_t lds[];
@@ -642,7 +630,7 @@ __global__ __launch_bounds__(kNW * kWave) void sparse_mla_kernel(MlaArgs a) {
   const int b = bs_row / a.S;
   const int s = bs_row % a.S;
   // A wave owns two 16-head blocks: heads head0 + 16*hb + r.
-  const int head0 = blockIdx.y * (kNW * kHeadsPerWave) + wave * kHeadsPerWave;
+  const int head0 = blockIdx.y * (kMlaWaves * kHeadsPerWave) + wave * kHeadsPerWave;
   bool hb_on[2];
   hb_on[0] = head0 < a.H;
   hb_on[1] = head0 + 16 < a.H;
@@ -664,7 +652,7 @@ __global__ __launch_bounds__(kNW * kWave) void sparse_mla_kernel(MlaArgs a) {
   // Every load below is issued unconditionally, from a clamped valid address
   // (its value is discarded later if out of range): conditional loads would
   // make the compiler wait for them on the spot.
-  constexpr int kIdxPerLane = kSlotsCap / (kNW * kWave);  // slot indices a lane may translate
+  constexpr int kIdxPerLane = kSlotsCap / (kMlaWaves * kWave);  // slot indices a lane may translate
   const int last_slot = max(min(slot_end, a.topk) - 1, 0);  // clamped: slot_end may be 0
   int idx_raw[kIdxPerLane];
 #pragma unroll
@@ -866,7 +854,7 @@ __global__ __launch_bounds__(kNW * kWave) void sparse_mla_kernel(MlaArgs a) {
     // first MFMA.  Iteration t sends tile t + kDepth while it exists.
 #pragma unroll
     for (int t = 0; t < kDepth; ++t) {
-      TileDma<kNW, kD> dma;
+      TileDma<kD> dma;
       dma.prepare(kvb, kvb2, trows, safe_row, min(t, ntiles - 1), lds + (t % kStages) * kStageBytes, wave, lane);
       il_dma_all(dma);
     }
@@ -877,8 +865,8 @@ __global__ __launch_bounds__(kNW * kWave) void sparse_mla_kernel(MlaArgs a) {
       f32x4 c[2][2];
       uint32_t qa[2];
       stage_k(0, qa);
-      TileDma<kNW, kD> none;
-      qk_phase<kF16, kNW, kD, false>(c, qb, qa, none);
+      TileDma<kD> none;
+      qk_phase<kF16, kD, false>(c, qb, qa, none);
       mask_scores(c, __builtin_amdgcn_readfirstlane(tmask[0]));
       // The first processed tile holds the first valid slot: it fixes m_ref.
 #pragma unroll
@@ -907,7 +895,7 @@ __global__ __launch_bounds__(kNW * kWave) void sparse_mla_kernel(MlaArgs a) {
       constexpr bool kDma = decltype(dma_c)::value;
       // The DMA of tile + kDepth (into the stage tile - 1 left) goes out
       // spread over phase A.
-      TileDma<kNW, kD> dma;
+      TileDma<kD> dma;
       if constexpr (kDma)
         dma.prepare(kvb, kvb2, trows, safe_row, tile + kDepth, lds + ((tile + kDepth) % kStages) * kStageBytes, wave,
                     lane);
@@ -915,7 +903,7 @@ __global__ __launch_bounds__(kNW * kWave) void sparse_mla_kernel(MlaArgs a) {
       uint32_t qa[2], va[2];
       stage_k(tile + 1, qa);
       stage_v(tile, va);
-      qk_phase<kF16, kNW, kD, kDma>(c, qb, qa, dma);
+      qk_phase<kF16, kD, kDma>(c, qb, qa, dma);
       mask_scores(c, __builtin_amdgcn_readfirstlane(tmask[tile + 1]));
       u32x4 pa_next[2];
       Softmax sm{c, pa_next, lsum, lsum_r, overflow, {-m_ref[0], -m_ref[1]}, scale_log2, {}};
@@ -964,8 +952,8 @@ __global__ __launch_bounds__(kNW * kWave) void sparse_mla_kernel(MlaArgs a) {
   if (*overflow_flag) {
     mla_exact_fallback<kF16, kD>(a.q, kvb, kvb2, sinks, obase, obase32, lbase, a.H, a.scale_log2, rows, nslots_all,
                                  token,
-                                 blockIdx.y * (kNW * kHeadsPerWave), kNW * kHeadsPerWave,
-                                 reinterpret_cast<float*>(lds), kNW * kWave);
+                                 blockIdx.y * (kMlaWaves * kHeadsPerWave), kMlaWaves * kHeadsPerWave,
+                                 reinterpret_cast<float*>(lds), kMlaWaves * kWave);
     return;
   }
 
@@ -1081,7 +1069,7 @@ __global__ __launch_bounds__(kNW * kWave) void sparse_mla_kernel(MlaArgs a) {
 // heads a workgroup (two workgroups per CU): window + 512 selected, 4096 rows,
 // 423 -> 355 and 429 -> 368 us; window alone, 8192 rows, 309 -> 206 and 330 -> 243;
 // 64 decode rows 57 -> 50 and 59 -> 51 (bit-equal too).
-constexpr int kR4Waves = 4;
+constexpr int kR4Waves = kMlaWaves;
 constexpr int kR4Heads = 64;                            // heads per workgroup
 constexpr int kR4PBytes = kR4Waves * 1024;              // one P operand per wave
 constexpr int kR4POffset = MlaLayout<512, 2>::kLds;
@@ -1110,10 +1098,10 @@ __device__ __forceinline__ void r4_k_first(u32x4 (&k)[kR4Ahead + 1], const uint3
 // by the parity of the step (the sums of qk_half).
 template <bool kF16, int kD, int kSets, bool kDma, int J>
 __device__ __forceinline__ void r4_qk(f32x4 (&c)[kSets][2], const u32x4 (&qb)[kD / 32], const uint32_t (&qa)[2],
-                                      u32x4 (&k)[kR4Ahead + 1], TileDma<kR4Waves, kD>& dma) {
+                                      u32x4 (&k)[kR4Ahead + 1], TileDma<kD>& dma) {
   constexpr int kHalf = MlaGeom<kD>::kQkHalf;
   if constexpr (J + kR4Ahead < kHalf) r4_k_read<J + kR4Ahead>(k, qa);
-  if constexpr (kDma) il_dma<kR4Waves, kD, J>(dma);
+  if constexpr (kDma) il_dma<kD, J>(dma);
   constexpr int kWait = (kHalf - 1 - J) < kR4Ahead ? (kHalf - 1 - J) : kR4Ahead;
   u32x4& kj = k[J % (kR4Ahead + 1)];
   lgkm_wait_k<kWait>(kj);
@@ -1237,7 +1225,7 @@ void sparse_mla_rows4_kernel(MlaArgs a) {
   const uint32_t p_base = lds_u32(lds + kR4POffset) + 16 * lane;
 
   if (ntiles > 0) {
-    TileDma<kR4Waves, 512> dma;
+    TileDma<512> dma;
     dma.prepare(kvb, kvb2, trows, safe_row, 0, lds, wave, lane);
     il_dma_all(dma);
   }
@@ -1247,7 +1235,7 @@ void sparse_mla_rows4_kernel(MlaArgs a) {
     wait_vmcnt<0>();
     raw_barrier();
     const bool more = tile + 1 < ntiles;  // workgroup-uniform
-    TileDma<kR4Waves, 512> dma;
+    TileDma<512> dma;
     if (more) dma.prepare(kvb, kvb2, trows, safe_row, tile + 1, lds + ((tile + 1) & 1) * kStageBytes, wave, lane);
     const uint32_t mask = __builtin_amdgcn_readfirstlane(tmask[tile]);
     const uint32_t base = lds_u32(lds + (tile & 1) * kStageBytes);
@@ -1527,7 +1515,7 @@ void sparse_mla_heads64_kernel(MlaArgs a) {
       idx_nn = load_idx(kStages);
 #pragma unroll
       for (int t = 0; t < kStages; ++t) blk[t] = load_blk(idx[t]);
-      TileDma<kR4Waves, kD> dma;
+      TileDma<kD> dma;
       dma.prepare_src(lane_src(0, idx[0], blk[0]), lds, wave);
       il_dma_all(dma);
     }
@@ -1537,7 +1525,7 @@ void sparse_mla_heads64_kernel(MlaArgs a) {
     if (ntiles > 0) {
       if constexpr (kDepth == 2) {
         __asm__ __volatile__("" ::: "memory");
-        TileDma<kR4Waves, kD> dma;
+        TileDma<kD> dma;
         dma.prepare_src(lane_src(1, idx[1], blk[1]), lds + kStageBytes, wave);
         il_dma_all(dma);
       }
@@ -1567,7 +1555,7 @@ void sparse_mla_heads64_kernel(MlaArgs a) {
     wait_vmcnt<(kDepth - 1) * kTileLoads>();
     raw_barrier();
     // Past the last tile every slot is empty: the zero row, into a stage no one reads.
-    TileDma<kR4Waves, kD> dma;
+    TileDma<kD> dma;
     dma.prepare_src(lane_src(tile + kDepth, idx_n, blk_n), lds + fill, wave);
     blk_n = load_blk(idx_nn);
     // A move of its own: one the compiler places may come after the load below and wait for it.
@@ -1886,10 +1874,10 @@ hipError_t mla_scratch_ptr(void** out) {
 template <bool kF16, int kD, bool kPaged>
 static hipError_t launch_mla_kernel(const MlaArgs& a, int head_groups, hipStream_t stream) {
   const dim3 grid((unsigned)((int64_t)a.B * a.S * a.G * a.splits), (unsigned)head_groups);
-  constexpr int kNW = 4, kLds = MlaLayout<kD, kStages>::kLds;
-  const hipError_t e = set_dynamic_lds_once<sparse_mla_kernel<kNW, kF16, kD, kPaged>>(kLds);
+  constexpr int kLds = MlaLayout<kD, kStages>::kLds;
+  const hipError_t e = set_dynamic_lds_once<sparse_mla_kernel<kF16, kD, kPaged>>(kLds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((sparse_mla_kernel<kNW, kF16, kD, kPaged>), grid, dim3(kNW * kWave), kLds, stream, a);
+  hipLaunchKernelGGL((sparse_mla_kernel<kF16, kD, kPaged>), grid, dim3(kMlaWaves * kWave), kLds, stream, a);
   return hipGetLastError();
 }
 
