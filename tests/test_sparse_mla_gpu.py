@@ -196,8 +196,8 @@ def _ring_depth(dsa, B, S, H, topk):
 
 @pytest.mark.parametrize("B,S,H,topk,paged,stages", [
     (1, 9, 16, 31, False, 2), (3, 3, 48, 1100, True, 2), (2, 130, 64, 33, True, 2), (120, 1, 32, 1100, True, 2),
-    (1, 120, 64, 1088, False, 2), (1, 300, 48, 2049, False, 2), (1, 128, 64, 2048, False, 3), (2, 64, 16, 2048, True, 3),
-    (1, 256, 48, 1100, False, 3), (2, 128, 64, 545, True, 3)])
+    (1, 120, 64, 1088, False, 2), (1, 300, 48, 2049, False, 2), (1, 128, 64, 2048, False, 3),
+    (2, 64, 16, 2048, True, 3), (1, 256, 48, 1100, False, 3), (2, 128, 64, 545, True, 3)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_up_to_64_heads_tile_and_stage_edges(dsa, dev, B, S, H, topk, paged, stages, dtype):
     """The 64-head kernel: both ring depths, splits, ragged last tiles, empty tiles, heads short of 64.
@@ -280,8 +280,8 @@ def test_decode_rows_read_no_key_for_empty_slots(dsa, dev, T, topk, form):
     if apart:
         cut = lambda t: (t[..., :512].contiguous().to(dev), t[..., 512:].contiguous().to(dev))  # noqa: E731
         (ql, qr), (kc, kr) = cut(q[0]), cut(src)
-        out = dsa.sparse_attn_tilelang(ql, kc, kc, idx[0].to(dev), 0.05, 1, None, kl.to(dev), query_rope=qr, key_rope=kr,
-                                       sparse_mode=3, **kw)
+        out = dsa.sparse_attn_tilelang(ql, kc, kc, idx[0].to(dev), 0.05, 1, None, kl.to(dev), query_rope=qr,
+                                       key_rope=kr, sparse_mode=3, **kw)
         torch.testing.assert_close(out[None].float().cpu(), want, atol=2e-2, rtol=2e-2)
     else:
         out, lse = dsa.sparse_mla_fwd(q.to(dev), src.to(dev), idx.to(dev), 0.05, actual_seq_lengths_kv=kl.to(dev), **kw)
