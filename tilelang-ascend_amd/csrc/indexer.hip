@@ -235,9 +235,10 @@ __device__ __forceinline__ u32x4 relu_operand(const f32x4& c0, const f32x4& c1) 
 
 // Head reduction of more than 32 heads by one structured-sparse MFMA: D +=
 // W * relu(scores) over K = 64 heads in the cycles a dense 16x16x32 takes for 32
-// (the dense pair took a fifth of the matrix cycles, and these passes run at the
-// card's power limit: 4096 rows x 32768 keys with top-2048 990 -> 960 us, x 131072
-// keys 3550 -> 3370 us).  W has at most two weights in every four K: even rows hold heads 4m, 4m + 1 of each four, odd rows heads 4m + 2, 4m + 3
+// (the dense pair took a fifth of the matrix cycles, of which these passes keep the
+// matrix cores busy 70%: calls of 4096 rows x 32768 keys with top-2048 929 -> 883
+// us, x 131072 keys 3506 -> 3300 us).  W has at most two weights in every four K:
+// even rows hold heads 4m, 4m + 1 of each four, odd rows heads 4m + 2, 4m + 3
 // (sparse_index), so a logit is the sum of an even and an odd row.  Rows 4n + 2j
 // and 4n + 2j + 1 belong to the wave's token j: both tokens accumulate into one D,
 // whose components 2j, 2j + 1 in every lane are token j's halves for key r.
@@ -257,7 +258,8 @@ __device__ __forceinline__ f32x4 sparse_sum(const u32x4& w, const f32x4& c0, con
 
 // Sums over the four lane groups of four values per lane: lane group g gets the sum of x[g].  Three
 // swaps and three adds on the VALU for a token's 64 keys, where each 16-key slice took two LDS
-// shuffles and a select (packed bf16 rows, 24 heads, top-2048 included: 560 -> 523 us).
+// shuffles and a select (three packed batches of 340 to 1699 bf16 rows of 24 heads by 3000 to 15000
+// keys, top-2048 included: 534 -> 502 us).
 __device__ __forceinline__ float group_sums(const float (&x)[4]) {
   // permlane32_swap(a, b): {a.lo, b.lo} and {a.hi, b.hi}; permlane16_swap the same by odd and even groups.
   auto add32 = [](float a, float b) {
@@ -942,9 +944,9 @@ static IdxArgs make_idx_args(const void* q, const void* k, const float* k_scale,
 
 // Keys per workgroup.  3072 workgroups are four whole rounds of the three a CU
 // holds, and level out batches of unequal lengths, whose grid spans the longest
-// (packed bf16 rows of 340 to 1699 queries by 3000 to 15000 keys: 523 -> 464 us
-// against 2048 workgroups; 4096 rows by 8192 keys 322 -> 311; 4096 and more
-// workgroups gain nothing further and cost the latter 10%).  split: one token
+// (against 2048 workgroups, top-2048 included: three packed batches of 340 to 1699
+// bf16 rows by 3000 to 15000 keys 502 -> 444 us, 4096 fp8 rows by 8192 keys 302 ->
+// 281; 4096 and more workgroups gain nothing further and cost the latter 10%).  split: one token
 // per workgroup (dense logits of few query rows), 2048: their chunks are short
 // already (32 rows by 131072 keys).
 static int64_t indexer_key_chunk(int64_t B, int64_t S1, int64_t S2, bool split = false) {

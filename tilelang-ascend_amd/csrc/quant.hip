@@ -10,8 +10,8 @@
 //
 // Aligned rows of up to 2048 16-byte chunks (act_quant_rows_kernel): a row is held in the registers
 // of a group of lanes, as many as it has chunks (up to the wave), so the 256-byte rows of a 128-wide
-// head fill the wave four at a time and are read once: 262144 bf16 rows of 128 take 17.6 us (5.8 TB/s)
-// against 84.0 with a wave per row, where 16 of 64 lanes loaded; 4681 rows of 7168 23.7 against 31.6.  Other rows (act_quant_kernel): one wave per
+// head fill the wave four at a time and are read once: 262144 bf16 rows of 128 take 17.4 us (5.8 TB/s)
+// against 84.2 with a wave per row, where 16 of 64 lanes loaded; 4681 rows of 7168 23.7 against 31.6.  Other rows (act_quant_kernel): one wave per
 // row, a pass for the absolute maximum and a pass that scales, converts and stores.
 #include "common.hpp"
 

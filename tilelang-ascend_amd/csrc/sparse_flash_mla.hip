@@ -886,7 +886,16 @@ static hipError_t launch_v4_decode_rows(int is_fp16, const void* q, const void* 
 // Sparse MLA (576-wide rows, V = the first 512) decode rows through the decode
 // kernel: at most kDecodeRows query rows, at most 1024 (row, head) pairs (so the
 // partials stay within the allocation-free entry's scratch), at most
-// kMlaDecodeMaxSlots index slots.
+// kMlaDecodeMaxSlots index slots.  Both sides measured, us a call (paged caches of
+// 64K tokens; this kernel | the gather kernels):
+//   512 slots, 1 / 8 rows: 64 heads 13.4 / 15.1 | 16.5 / 17.4, 128 heads 13.6 / 17.5 | 22.0 / 23.7;
+//   2048 slots, 16 heads, 1 / 8 rows: 16.7 / 18.8 | 15.7 / 17.4;
+//   64 heads, 1 / 4 / 5 / 8 rows: 17.5 / 19.9 / 29.3 / 29.2 | 18.6 / 19.9 / 20.7 / 22.5;
+//   128 heads, 1 / 2 / 3 / 8 rows: 18.8 / 20.2 / 30.4 / 48.0 | 24.4 / 25.2 / 26.4 / 30.2.
+// So the line is not the crossover, which lies where the grid (rows x heads / 16 x
+// chunks, one workgroup per CU) passes 256 workgroups: the larger calls stay here
+// because parts that lie apart have this kernel alone, and both entries give the
+// same bits.
 constexpr int64_t kMlaDecodeMaxSlots = 2048;
 
 bool mla_decode_applies(int64_t T, int64_t H, int64_t topk) {
